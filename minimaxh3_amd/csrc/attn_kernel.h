@@ -20,12 +20,13 @@
 // a lane-constant 0/1 selector as A (AttnFragOfs::rowsum_sel).  K and V^T tiles (and the
 // mask / bias of the tile) are copied global -> LDS by the direct-to-LDS DMA.
 //
-// Per score the VALU does half a 3-input max and three FMAs ((8 S + 56 - 8 m) / 8 straight
-// from the fp32 dot product with the per-tile constant sq sk; the flush test as a clamped
-// FMA; rounding to an integer code by adding 1.5 * 2^20), plus three quarters of a byte
-// permute to pack the codes.  Folding sq * sk into one constant rounds 8 S once instead of
-// twice; the row max that drives the lazy-max policy is still computed exactly as
-// (max * sq) * sk.
+// Per score the VALU does half a 3-input max, one FMA and one multiply: the FMA makes
+// 8 S + 56 - 8 m straight from the fp32 dot product, scaled so that the flush of codes below
+// 8 is the hardware's flush of denormal results, and the multiply rounds it to the integer
+// code, as the bit pattern of a denormal, into its byte of the packed codes
+// (attn_codes_tile; the repair keeps a form of its own, attn_codes_w4).  Folding sq * sk
+// into one constant rounds 8 S once instead of twice; the row max that drives the lazy-max
+// policy is still computed exactly as (max * sq) * sk.
 //
 // The repair correction delta = exp2(S - m) - P (where P >= tau) is formed from the same
 // bits and split into two e4m3 parts of 8 delta that the PV products multiply with the V^T
@@ -363,12 +364,14 @@ struct AttnState {
   // (see AttnMfmaRun, x == NDT).
   v4f lacc;
   float m;  // lazy row max (log2 domain)
-  // the code constants that depend on m (see attn_codes_w4): 7 - m and (48 - 8 m) 2^64
-  float cst8, cstf;
+  // the code constants that depend on m: (7 - m) 2^-126 (attn_codes_tile), and with the
+  // repair 7 - m and (48 - 8 m) 2^64 (attn_codes_w4)
+  float csty, cst8, cstf;
 
   __device__ __forceinline__ void set_m(float m_new) {
     m = m_new;
     cst8 = 7.0f - m_new;
+    csty = cst8 * 0x1p-126f;
     cstf = (48.0f - 8.0f * m_new) * 0x1p64f;
   }
 
@@ -459,7 +462,93 @@ struct AttnPB {
   v8i lo[REP ? 2 : 1];
 };
 
-// Per-tile constants of the code arithmetic (see attn_codes_w4).
+// Whether the score products run at the block scale 2^-96 (kScoreScaleE8M0): the codes
+// without the repair are made from scores near the bottom of the fp32 range
+// (attn_codes_tile), where a score cannot be brought by a constant of the FMA (sq sk 2^-126 is
+// no normal number).  The scale only shifts exponents: every product and sum keeps its
+// significand.  With a bias the score is formed from dot, sq and sk one by one, unscaled.
+template <bool HAS_BIAS, bool REP>
+constexpr bool attn_scores_scaled() {
+  return !HAS_BIAS && !REP;
+}
+constexpr int kScoreScaleE8M0 = 127 - 96;
+constexpr float kScoreScale = 0x1p-96f;
+
+// Single-precision denormals of this wave's VALU (MODE bits 5:4): bit 0 lets denormal inputs
+// through, bit 1 denormal results.  (Volatile asm, which stays in order with the asm
+// statements between two calls; the builtin's instruction may move across them.)
+template <int BITS>
+__device__ __forceinline__ void set_f32_denorm() {
+  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 4, 2), %0" ::"n"(BITS));
+}
+
+// The exp2-free P codes of one tile without the repair: word 4 (t & 1) + w4 of the PV B
+// operand of key half t >> 1 holds scores 4 w4 .. 4 w4 + 3 of subtile t.
+//
+// code = bits < 8 ? 0 : rint(bits), bits = 8 S + 56 - 8 m.  bits never exceeds 8 * 8 + 56 =
+// 120 (the lazy max keeps S <= m + 8), so the reference's clamp to [0, 126] is inactive.
+//   y    = clamp01(fma(x, cy, csty)) = max(bits, 0) 2^-129, flushed to 0 below 2^-126
+//   code = y 2^-20 as a denormal, whose bit pattern is rint(bits)
+// x cy = 2^-126 S (x the score scaled by 2^-96 and cy = sq sk 2^-30, or x = S and cy = 2^-126
+// with a bias) and csty = (7 - m) 2^-126.  bits = 8 is the smallest normal number there, so
+// with denormal results flushed (denormal inputs stay: csty is one for m near 7) the FMA
+// itself makes bits < 8 zero, its output clamp the negative ones (masked keys too), and
+// a normal result is rounded as bits itself would be: RN(bits) 2^-129.  With denormal results
+// allowed again the multiply leaves multiples of 2^-149, rounded to nearest even, in one byte
+// of the word (the SDWA form keeps the other three).
+//
+// Two VALU instructions per score and no packing.  The instruction rates this follows,
+// measured on MI355X (two waves per SIMD, cycles per wave instruction at 2.4 GHz): FMA 3.1,
+// add 2.7, multiply into a byte 4.7, v_perm_b32 / v_max3 4.6.  The form it replaces here (three
+// FMAs and 3/4 of a permute or OR per score) took 12.7 cycles against 7.8; codes compared
+// bit for bit over 10^8 scores, boundaries of the flush among them (where exact bits below 8
+// round to 8 the code is now 8, as the reference's test of the rounded value gives).
+//
+// The instructions are volatile asm, which keeps them between the two mode changes and in
+// this order: a word's next byte is written four instructions after the last (one wait state
+// is needed), and the s_nop at the end covers the last write before a matrix product reads
+// the words.  Every score was read by attn_part_max before, so none is still
+// being written by a matrix product.
+template <bool HAS_BIAS>
+__device__ __forceinline__ void attn_codes_tile(const v16f (&s)[4], float sq, float skj, float csty, v8i (&p)[2]) {
+  float cy = HAS_BIAS ? 0x1p-126f : (sq * skj) * (0x1p-126f / kScoreScale);
+  float cr = 0x1p-20f;
+  float y[4][16];
+  asm volatile("" : "+v"(cy), "+v"(csty), "+v"(cr));
+  set_f32_denorm<1>();
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      asm volatile("v_fma_f32 %0, %1, %2, %3 clamp" : "=v"(y[t][i]) : "v"(s[t][i]), "v"(cy), "v"(csty));
+  set_f32_denorm<3>();
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    uint32_t w[4];
+    const float(&u)[16] = y[t];
+#define MXF8_MUL_BYTE(B, W, Y) \
+  "v_mul_f32_sdwa %" #W ", %4, %" #Y " dst_sel:BYTE_" #B " dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD\n"
+    asm volatile(
+        "v_mul_f32 %0, %4, %5\n"
+        "v_mul_f32 %1, %4, %9\n"
+        "v_mul_f32 %2, %4, %13\n"
+        "v_mul_f32 %3, %4, %17\n"
+        // clang-format off
+        MXF8_MUL_BYTE(1, 0, 6) MXF8_MUL_BYTE(1, 1, 10) MXF8_MUL_BYTE(1, 2, 14) MXF8_MUL_BYTE(1, 3, 18)
+        MXF8_MUL_BYTE(2, 0, 7) MXF8_MUL_BYTE(2, 1, 11) MXF8_MUL_BYTE(2, 2, 15) MXF8_MUL_BYTE(2, 3, 19)
+        MXF8_MUL_BYTE(3, 0, 8) MXF8_MUL_BYTE(3, 1, 12) MXF8_MUL_BYTE(3, 2, 16) MXF8_MUL_BYTE(3, 3, 20)
+        // clang-format on
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3])
+        : "v"(cr), "v"(u[0]), "v"(u[1]), "v"(u[2]), "v"(u[3]), "v"(u[4]), "v"(u[5]), "v"(u[6]), "v"(u[7]), "v"(u[8]),
+          "v"(u[9]), "v"(u[10]), "v"(u[11]), "v"(u[12]), "v"(u[13]), "v"(u[14]), "v"(u[15]));
+#undef MXF8_MUL_BYTE
+#pragma unroll
+    for (int w4 = 0; w4 < 4; ++w4) p[t >> 1][4 * (t & 1) + w4] = (int)w[w4];
+  }
+  asm volatile("s_nop 3");
+}
+
+// Per-tile constants of the code arithmetic with the repair (see attn_codes_w4).
 struct AttnCodeK {
   float c1, cst8, c8f, cstf;
   uint32_t rep_add;  // the repair threshold as a byte addend (attn_repair_addend)
@@ -495,12 +584,9 @@ static inline uint32_t attn_repair_addend(float tau) {
   return (uint32_t)(0x80 - T) * 0x01010101u;
 }
 
-// The exp2-free P codes of scores 4 w4 .. 4 w4 + 3 of score subtile t: word 4 (t & 1) + w4
-// of the PV B operand of key half t >> 1.
-//
-// code = bits < 8 ? 0 : rint(bits), bits = 8 S + 56 - 8 m_new.  bits never exceeds
-// 8 * 8 + 56 = 120 (the lazy max keeps S <= m + 8), so the reference's clamp to [0, 126] is
-// inactive.  Three FMAs per score, all at the full FMA rate, on b = bits / 8 (exactly: an
+// The codes of attn_codes_tile for the repair, which needs bits / 8 itself in its normal
+// range for the exact exp2, and the two parts of its correction: scores 4 w4 .. 4 w4 + 3 of
+// score subtile t.  Three FMAs per score, all at the full FMA rate, on b = bits / 8 (exactly: an
 // eighth of every term, so b = RN(bits) / 8):
 //   b    = fma(dot, c1, cst8)                                (c1 = sq sk, cst8 = 7 - m)
 //   keep = clamp01(fma(dot, 8 c1 2^64, (48 - 8 m) 2^64))     (1 when bits >= 8, else 0)
@@ -512,7 +598,7 @@ static inline uint32_t attn_repair_addend(float tau) {
 // leaves rint(bits) in the low mantissa bits of t (0 when keep is 0), so v_perm_b32 packs the
 // low bytes of four t's into one dword of codes.
 //
-// Repair (REP, kernels/fp8_attention.py:288-292): delta = exp2(S - m) - P where P >= tau,
+// Repair (kernels/fp8_attention.py:288-292): delta = exp2(S - m) - P where P >= tau,
 // else 0.  exp2(b) = exp2(S - m + 7) = 128 exp2(S - m); P is the decoded code.  delta is
 // bounded by about 11% of exp2(S - m) <= 2^8 (the code's relative error: Mitchell's 6.1% and
 // the rounding of bits), so |8 delta| < 448 and 8 delta splits into e4m3 parts
@@ -522,8 +608,7 @@ static inline uint32_t attn_repair_addend(float tau) {
 // 8 delta, and decoded values 16 times theirs).  hi + lo holds 8 delta to about 8
 // significant bits (exactly its bf16 rounding's precision for |8 delta| >= 2^-2; below that
 // lo's e4m3 grid, 2^-9, bounds the error), where the reference rounds delta to bf16.
-template <bool REP>
-__device__ __forceinline__ void attn_codes_w4(const v16f& st, const AttnCodeK& k, int t, int w4, AttnPB<REP>& pb) {
+__device__ __forceinline__ void attn_codes_w4(const v16f& st, const AttnCodeK& k, int t, int w4, AttnPB<true>& pb) {
   {
     uint32_t tb[4];
     float b8[4];
@@ -541,7 +626,7 @@ __device__ __forceinline__ void attn_codes_w4(const v16f& st, const AttnCodeK& k
     // (the PV products): a reordered tile would hold the scores and the codes live together.
     asm volatile("" ::"v"(word));
     pb.p[t >> 1][4 * (t & 1) + w4] = (int)word;
-    if constexpr (REP) {
+    {
       const v2f p01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)word, false);
       const v2f p23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)word, true);
       const float papx[4] = {p01[0], p01[1], p23[0], p23[1]};
@@ -567,21 +652,14 @@ __device__ __forceinline__ void attn_codes_w4(const v16f& st, const AttnCodeK& k
   }
 }
 
-// The codes of score subtile t.
-template <bool REP>
-__device__ __forceinline__ void attn_codes_sub(const v16f& st, const AttnCodeK& k, int t, AttnPB<REP>& pb) {
-#pragma unroll
-  for (int w4 = 0; w4 < 4; ++w4) attn_codes_w4<REP>(st, k, t, w4, pb);
-}
-
 // A run of matrix-core products with their A fragments fetched from LDS AHEAD products
 // ahead (AHEAD + 1 fragments in flight), so the products issue back to back instead of
 // each waiting for its own LDS read.  The run is the PV products of key halves
 // [KH0, KH1) of one tile (per half: O^T tile x for x < D/32, then the row-sum product at
 // x == D/32; with REP each fragment also multiplies the two repair parts) followed by the
 // QK^T products of score subtiles [U0, U1) of another (per subtile: the D/64 channel
-// halves hh).
-template <int D, int KH0, int KH1, int U0, int U1, int AHEAD = 3>
+// halves hh), at the block scale KSC of K (127 = 1.0).
+template <int D, int KH0, int KH1, int U0, int U1, int KSC = 127, int AHEAD = 3>
 struct AttnMfmaRun {
   static constexpr int RING = AHEAD + 1;
   static constexpr int NDT = D / 32, QKM = D / 64;
@@ -599,6 +677,13 @@ struct AttnMfmaRun {
       constexpr int u = U0 + (K - NPV) / QKM, hh = (K - NPV) % QKM;
       return lds_pair(sK + u * 32 * D, fo.k[hh][0], fo.k[hh][1]);
     }
+  }
+
+  __device__ static __forceinline__ v16f qk(const v8i& kf, const v8i& qf, const v16f& c) {
+    if constexpr (KSC == 127)
+      return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kf, qf, c, 0, 0, 0, 0, 0, 0);
+    else
+      return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kf, qf, c, 0, 0, 0, KSC, 0, 127);
   }
 
   template <int K, bool REP>
@@ -629,9 +714,9 @@ struct AttnMfmaRun {
         v16f z;
 #pragma unroll
         for (int i = 0; i < 16; ++i) z[i] = 0.0f;
-        s[u] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fr, qf[0], z, 0, 0, 0, 0, 0, 0);
+        s[u] = qk(fr, qf[0], z);
       } else {
-        s[u] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fr, qf[hh], s[u], 0, 0, 0, 0, 0, 0);
+        s[u] = qk(fr, qf[hh], s[u]);
       }
     }
   }
@@ -671,13 +756,14 @@ struct AttnMfmaRun {
 };
 
 // Score given to invalid keys: finite and so negative that it loses every row max and
-// flushes to code 0.  The flush test multiplies it by c8 = 8 sq sk (or 8 with a bias), so
+// flushes to code 0.  The codes multiply it by c8 = 8 sq sk (or 8 with a bias), so
 // it is chosen to make that product -1e30 (finite: no inf * 0 = NaN downstream); for
-// c8 < 1e-8 it is -1e38 and the product is smaller still.
-template <bool HAS_BIAS>
+// c8 < 1e-8 it is -1e38 and the product is smaller still.  SC: at the scale of the scores.
+template <bool HAS_BIAS, bool SC>
 __device__ __forceinline__ float attn_invalid_score(float sq, float skj) {
   if constexpr (HAS_BIAS) return -1.25e29f;
-  return -1.0e30f / fmaxf((8.0f * sq) * skj, 1.0e-8f);
+  const float v = -1.0e30f / fmaxf((8.0f * sq) * skj, 1.0e-8f);
+  return SC ? v * kScoreScale : v;
 }
 
 // Whether tile [kv0, kv0 + 128) has any invalid key (wave-uniform).  A bias applies to
@@ -721,14 +807,13 @@ __device__ __forceinline__ float attn_bias_score(float dot, float sq, float skj,
 
 // Invalid keys (past Sk, masked, bias <= -1e8) get attn_invalid_score; with a bias S is
 // formed explicitly as (dot * sq) * sk + bias * log2 e.
-// Score subtiles [T0, T0 + NT).
-template <bool HAS_MASK, bool HAS_BIAS, int T0 = 0, int NT = 4>
+template <bool HAS_MASK, bool HAS_BIAS, bool SC>
 __device__ __forceinline__ void attn_mask_scores(v16f (&s)[4], const uint8_t* sAux, int kv0, int Sk, float sq,
                                                  float skj, int lane) {
   const int g = lane >> 5;
-  const float vinv = attn_invalid_score<HAS_BIAS>(sq, skj);
+  const float vinv = attn_invalid_score<HAS_BIAS, SC>(sq, skj);
 #pragma unroll
-  for (int t = T0; t < T0 + NT; ++t) {
+  for (int t = 0; t < 4; ++t) {
     const int kb = 64 * (t >> 1) + 16 * (t & 1) + 32 * g;
     float bias[16];
     if constexpr (HAS_BIAS) {
@@ -757,14 +842,14 @@ __device__ __forceinline__ void attn_mask_scores(v16f (&s)[4], const uint8_t* sA
   }
 }
 
-// Row max over score subtiles [T0, T0 + NT) (exactly the reference's fp32 S max over
-// those keys: x -> (x * sq) * sk is monotonic), floored at -1e9.  Four independent v_max3
-// chains, so that the VALU need not wait on each result.
-template <bool HAS_BIAS, int T0 = 0, int NT = 4>
+// Row max of the tile (exactly the reference's fp32 S max over those keys: x -> (x * sq) * sk
+// is monotonic, and undoing the scores' power-of-two scale, SC, is exact), floored at -1e9.
+// Four independent v_max3 chains, so that the VALU need not wait on each result.
+template <bool HAS_BIAS, bool SC>
 __device__ __forceinline__ float attn_part_max(const v16f (&s)[4], float sq, float skj) {
   float m4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
-  for (int t = T0; t < T0 + NT; ++t)
+  for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) m4[i & 3] = fmaxf(m4[i & 3], s[t][i]);
   float mx = fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3]));
@@ -777,6 +862,7 @@ __device__ __forceinline__ float attn_part_max(const v16f (&s)[4], float sq, flo
     const auto sw = __builtin_amdgcn_permlane32_swap(u, u, false, false);
     asm("v_max_f32 %0, %1, %2" : "=v"(mx) : "v"(__uint_as_float(sw[0])), "v"(__uint_as_float(sw[1])));
   }
+  if constexpr (SC) mx *= 1.0f / kScoreScale;
   return fmaxf(HAS_BIAS ? mx : (mx * sq) * skj, kAttnNeg);
 }
 
@@ -794,16 +880,22 @@ template <bool HAS_BIAS, bool REP, int D>
 __device__ __forceinline__ void attn_softmax_tile(const v16f (&s)[4], float sq, float skj, uint32_t rep_add,
                                                   bool rescale,
                                                   AttnState<D>& st, AttnPB<REP>& pb) {
-  const float rmax = attn_part_max<HAS_BIAS>(s, sq, skj);
+  const float rmax = attn_part_max<HAS_BIAS, attn_scores_scaled<HAS_BIAS, REP>()>(s, sq, skj);
   const bool moves = attn_max_moves(rmax, st.m);
   if (__builtin_amdgcn_ballot_w64(moves)) {
     const float m_new = moves ? rmax : st.m;
     if (rescale) st.rescale(__builtin_amdgcn_exp2f(st.m - m_new));
     st.set_m(m_new);
   }
-  const AttnCodeK k = AttnCodeK::make<HAS_BIAS>(sq, skj, st.cst8, st.cstf, rep_add);
+  if constexpr (REP) {
+    const AttnCodeK k = AttnCodeK::make<HAS_BIAS>(sq, skj, st.cst8, st.cstf, rep_add);
 #pragma unroll
-  for (int t = 0; t < 4; ++t) attn_codes_sub<REP>(s[t], k, t, pb);
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int w4 = 0; w4 < 4; ++w4) attn_codes_w4(s[t], k, t, w4, pb);
+  } else {
+    attn_codes_tile<HAS_BIAS>(s, sq, skj, st.csty, pb.p);
+  }
 }
 
 // The channel scales sv of head bh that this lane's output channels take (see attn_store).
@@ -1004,14 +1096,15 @@ void attn_fwd_kernel(const uint8_t* __restrict__ q8, const uint8_t* __restrict__
     const int kv0 = j * 128;
     v16f s[4];
     AttnPB<DO_REPAIR> pb;
-    AttnMfmaRun<D, 0, 0, 0, 4>::run(buf + T::KB, buf, fo, pb, cx.qf, s, st);
+    constexpr bool SC = attn_scores_scaled<HAS_BIAS, DO_REPAIR>();
+    AttnMfmaRun<D, 0, 0, 0, 4, SC ? kScoreScaleE8M0 : 127>::run(buf + T::KB, buf, fo, pb, cx.qf, s, st);
     if (attn_tile_needs_mask<HAS_MASK, HAS_BIAS>(buf + T::KB + T::VB, kv0, Sk, lane)) {
       // (tested here, where only tiles with a masked key pay for it)
       if (attn_tile_all_masked<HAS_MASK, HAS_BIAS>(buf + T::KB + T::VB, lane)) {
         j = jn;
         return;
       }
-      attn_mask_scores<HAS_MASK, HAS_BIAS>(s, buf + T::KB + T::VB, kv0, Sk, cx.sqI, skj, lane);
+      attn_mask_scores<HAS_MASK, HAS_BIAS, SC>(s, buf + T::KB + T::VB, kv0, Sk, cx.sqI, skj, lane);
     }
     attn_softmax_tile<HAS_BIAS>(s, cx.sqI, skj, rep_add, true, st, pb);
     AttnMfmaRun<D, 0, 2, 0, 0>::run(buf + T::KB, buf, fo, pb, cx.qf, s, st);
@@ -1183,7 +1276,8 @@ void attn_fwd_resident_kernel(const uint8_t* __restrict__ q8, const uint8_t* __r
         const int kv0 = j * 128;
         v16f s[4];
         AttnPB<false> pb;
-        AttnMfmaRun<D, 0, 0, 0, 4>::run(buf + T::KB, buf, fo, pb, cx.qf, s, st);
+        constexpr bool SC = attn_scores_scaled<HAS_BIAS, false>();
+        AttnMfmaRun<D, 0, 0, 0, 4, SC ? kScoreScaleE8M0 : 127>::run(buf + T::KB, buf, fo, pb, cx.qf, s, st);
         if (attn_tile_needs_mask<HAS_MASK, HAS_BIAS>(buf + T::KB + T::VB, kv0, Sk, lane)) {
           // (not on the last tile, under which the next item's Q rows load: the fetched
           // registers live across the branch would not fit)
@@ -1191,7 +1285,7 @@ void attn_fwd_resident_kernel(const uint8_t* __restrict__ q8, const uint8_t* __r
             j = j + 1 == nk ? 0 : j + 1;
             return;
           }
-          attn_mask_scores<HAS_MASK, HAS_BIAS>(s, buf + T::KB + T::VB, kv0, Sk, cx.sqI, skj, lane);
+          attn_mask_scores<HAS_MASK, HAS_BIAS, SC>(s, buf + T::KB + T::VB, kv0, Sk, cx.sqI, skj, lane);
         }
         // O and l are still zero on the first tile processed: rescaling them changes no bit
         attn_softmax_tile<HAS_BIAS>(s, cx.sqI, skj, 0u, i > 0, st, pb);
