@@ -233,6 +233,56 @@ __device__ __forceinline__ v4f quad4(const v16f& c, int q) {
   return v4f{c[4 * q], c[4 * q + 1], c[4 * q + 2], c[4 * q + 3]};
 }
 
+// Output values of accumulators x (registers 4 q .. 4 q + 3 of a block, whose LoRA branch is
+// lacc), packed as two bf16 pairs, with the reference's roundings: bf16 linear output, bf16
+// branch, bf16 branch * scale, bf16 sum; GELU-tanh acts on the bf16 result.  Values go
+// through them in pairs (bf16r2); the last rounding is the output packing itself.
+template <int ACT, bool LORA>
+__device__ __forceinline__ uint2 gemm_out_quad(const v4f x, int q, const v16f& lacc, float sam, const v4f& swq,
+                                               const v4f& bq, float lora_scale) {
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(x[e] * sam, swq[e], bq[e]);
+#pragma unroll
+  for (int h = 0; h < 4; h += 2) {
+    if constexpr (LORA || ACT == MXF8_ACT_GELU_TANH) bf16r2(v[h], v[h + 1]);
+    if constexpr (LORA) {
+      float b0 = lacc[4 * q + h], b1 = lacc[4 * q + h + 1];
+      bf16r2(b0, b1);
+      // scale 1 (the runtime folds alpha / rank into B): bf16(b * 1) = b, so the product
+      // and its rounding change no bit and are skipped
+      if (lora_scale != 1.0f) {
+        b0 *= lora_scale;
+        b1 *= lora_scale;
+        bf16r2(b0, b1);
+      }
+      v[h] += b0;
+      v[h + 1] += b1;
+      if constexpr (ACT == MXF8_ACT_GELU_TANH) bf16r2(v[h], v[h + 1]);
+    }
+    if constexpr (ACT == MXF8_ACT_GELU_TANH) {
+      v[h] = gelu_tanh_f32(v[h]);
+      v[h + 1] = gelu_tanh_f32(v[h + 1]);
+    }
+  }
+  return make_uint2(bf16x2(v[0], v[1]), bf16x2(v[2], v[3]));
+}
+
+// LoRA branch of one 32x32 output block on the bf16 MFMA from global memory: lacc^T[n][m] =
+// sum_j B[n][j] t[m][j].  brow / trow: this lane's rows of B and t, at column 8 (lane / 32).
+// UNROLL: rank steps whose loads may be in flight together.
+template <int UNROLL>
+__device__ __forceinline__ void lora_rows_mma(const uint16_t* brow, const uint16_t* trow, int r, v16f& lacc) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) lacc[i] = 0.0f;
+#pragma unroll UNROLL
+  for (int kk = 0; kk < r; kk += 16) {
+    const v8bf bo = *reinterpret_cast<const v8bf*>(brow + kk);
+    const v8bf to = *reinterpret_cast<const v8bf*>(trow + kk);
+    lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bo, to, lacc, 0, 0, 0);
+  }
+}
+
 // LM (LoRA mode): with lora_t [M, r] = bf16(x A^T) and lora_b [N, r] = B, the epilogue adds
 // the reference's LoRA branch bf16(bf16(t B^T) * lora_scale) to the bf16 linear output.
 // In LORA_LDS mode the t and B tiles (r <= 128: one or two 64-column chunks) are copied
@@ -441,7 +491,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_fp8_rowwise_kernel(
     // The LoRA branch of block (a, b) (zero without LoRA).
     auto lora_block = [&](int a, int b) {
       v16f lacc;
-      if constexpr (LM != LORA_NONE) {
+      if constexpr (LM == LORA_LDS) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) lacc[i] = 0.0f;
       }
@@ -451,48 +501,13 @@ __global__ __launch_bounds__(C::THREADS) void gemm_fp8_rowwise_kernel(
         if (nl == 2) lora_chunk_mma<C>(lch1, nl_ + (lane & 31), ml, g, lacc);
       } else if constexpr (LM == LORA_GLOBAL) {
         // LoRA up-projection on the bf16 MFMA from global memory (r > 128)
-        const uint16_t* brow = lora_b + (int64_t)min(n0 + nl_ + (lane & 31), N - 1) * lora_r + 8 * g;
-        const uint16_t* trow = lora_t + (int64_t)min(m0 + ml, M - 1) * lora_r + 8 * g;
-        for (int kk = 0; kk < lora_r; kk += 16) {
-          const v8bf bo = *reinterpret_cast<const v8bf*>(brow + kk);
-          const v8bf to = *reinterpret_cast<const v8bf*>(trow + kk);
-          lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bo, to, lacc, 0, 0, 0);
-        }
+        lora_rows_mma<1>(lora_b + (int64_t)min(n0 + nl_ + (lane & 31), N - 1) * lora_r + 8 * g,
+                      lora_t + (int64_t)min(m0 + ml, M - 1) * lora_r + 8 * g, lora_r, lacc);
       }
       return lacc;
     };
-    // Output values of accumulators x (registers 4 q .. 4 q + 3 of a block, whose LoRA
-    // branch is lacc), packed as two bf16 pairs.
     auto out_quad = [&](const v4f x, int q, const v16f& lacc, float sam, const v4f& swq, const v4f& bq) {
-      // the reference's roundings: bf16 linear output, bf16 branch, bf16 branch * scale,
-      // bf16 sum; GELU-tanh acts on the bf16 result.  Values go through them in pairs
-      // (bf16r2); the last rounding is the output packing itself.
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(x[e] * sam, swq[e], bq[e]);
-#pragma unroll
-      for (int h = 0; h < 4; h += 2) {
-        if constexpr (LM != LORA_NONE || ACT == MXF8_ACT_GELU_TANH) bf16r2(v[h], v[h + 1]);
-        if constexpr (LM != LORA_NONE) {
-          float b0 = lacc[4 * q + h], b1 = lacc[4 * q + h + 1];
-          bf16r2(b0, b1);
-          // scale 1 (the runtime folds alpha / rank into B): bf16(b * 1) = b, so the product
-          // and its rounding change no bit and are skipped
-          if (lora_scale != 1.0f) {
-            b0 *= lora_scale;
-            b1 *= lora_scale;
-            bf16r2(b0, b1);
-          }
-          v[h] += b0;
-          v[h + 1] += b1;
-          if constexpr (ACT == MXF8_ACT_GELU_TANH) bf16r2(v[h], v[h + 1]);
-        }
-        if constexpr (ACT == MXF8_ACT_GELU_TANH) {
-          v[h] = gelu_tanh_f32(v[h]);
-          v[h + 1] = gelu_tanh_f32(v[h + 1]);
-        }
-      }
-      return make_uint2(bf16x2(v[0], v[1]), bf16x2(v[2], v[3]));
+      return gemm_out_quad<ACT, LM != LORA_NONE>(x, q, lacc, sam, swq, bq, lora_scale);
     };
 
     // (KVS: every tile is staged -- the host checks the row alignment and that N is a multiple
@@ -740,6 +755,12 @@ __global__ __launch_bounds__(C::THREADS) void gemm_fp8_rowwise_kernel(
   }
 }
 
+}  // namespace mxf8
+
+#include "gemm_ring.h"
+
+namespace mxf8 {
+
 // ---- LoRA down-projection t = bf16(x A^T): x [M,K] bf16, A [r,K] bf16 -> t [M,r] -----
 // A workgroup computes BM = 32 W rows of t by up to 128 rank columns (blockIdx.y selects
 // columns [128 y, 128 y + 128)) on W waves of 32 rows, RT accumulators of 32 columns each.
@@ -943,9 +964,24 @@ extern "C" int mxf8_gemm_rowwise(const uint8_t* a8, const uint8_t* w8, const flo
   const uint16_t* lt = static_cast<const uint16_t*>(lora_t);
   const uint16_t* lb = static_cast<const uint16_t*>(lora_b);
   uint16_t* o16 = static_cast<uint16_t*>(out);
-  // 256x256 tiles when they fill the chip, 128x128 otherwise.
+  // 256x256 tiles when they fill the chip; below that the ring kernel where it is faster,
+  // 128x128 otherwise.
   const int64_t big_tiles = cdiv(M, 256) * cdiv(N, 256);
-  if (big_tiles >= 2 * 256)
+  const int cus = device_cus();
+  const int ring = big_tiles >= 2 * 256 || cus <= 0 ? -1 : gemm_ring_pick(M, N, K, lora ? r : 0, cus);
+  if (ring == 0)
+    launch_gemm_ring<GemmRing32x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
+                                    ld_out, stream);
+  else if (ring == 1)
+    launch_gemm_ring<GemmRing64x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
+                                    ld_out, stream);
+  else if (ring == 2)
+    launch_gemm_ring<GemmRing128x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
+                                     ld_out, stream);
+  else if (ring == 3)
+    launch_gemm_ring<GemmRing128x128>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
+                                      ld_out, stream);
+  else if (big_tiles >= 2 * 256)
     gemm_dispatch_tile<GemmBig>(act, lm, ktail, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
                                 ld_out, stream);
   else
