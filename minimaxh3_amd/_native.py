@@ -12,8 +12,10 @@ import threading
 import torch
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libmxf8.so")
+_OPS_PATH = os.path.join(os.path.dirname(_LIB_PATH), "libmxf8_torch.so")
 _lock = threading.Lock()
 _lib = None
+_ops_loaded = False
 
 BF16, F16, F32 = 0, 1, 2
 ACT_NONE, ACT_GELU_TANH = 0, 1
@@ -84,6 +86,19 @@ def load():
                     f"{_LIB_PATH} is missing: build the HIP library first (python -m minimaxh3_amd.build)")
             _lib = _bind(_LIB_PATH)
         return _lib
+
+
+def load_ops() -> None:
+    """Load libmxf8_torch.so once: the native kernels of the hot torch ops, over libmxf8."""
+    global _ops_loaded
+    load()
+    with _lock:
+        if not _ops_loaded:
+            if not os.path.exists(_OPS_PATH):
+                raise RuntimeError(
+                    f"{_OPS_PATH} is missing: build the HIP library first (python -m minimaxh3_amd.build)")
+            torch.ops.load_library(_OPS_PATH)
+            _ops_loaded = True
 
 
 def check(rc: int, what: str) -> None:

@@ -1,7 +1,9 @@
-"""Build recipe for the native library ``minimaxh3_amd/_lib/libmxf8.so`` (gfx950 only).
+"""Build recipe for the native libraries in ``minimaxh3_amd/_lib`` (gfx950 only).
 
 Each ``csrc/*.hip`` file is compiled by hipcc in parallel and the objects are linked into
-one shared library exporting the C ABI declared in ``include/mxf8.h``.
+one shared library, ``libmxf8.so``, exporting the C ABI declared in ``include/mxf8.h``.
+``csrc/torch_ops.cpp`` (host code: the hot torch ops over that ABI) becomes
+``libmxf8_torch.so``.
 
     python -m minimaxh3_amd.build            # build (always recompiles)
 """
@@ -11,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
@@ -18,6 +21,7 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 LIBDIR = os.path.join(PKG, "_lib")
 LIBNAME = "libmxf8.so"
+OPSNAME = "libmxf8_torch.so"
 # (source, object name, extra defines); attn_inst.hip is instantiated per (D, out dtype)
 SOURCES = [
     ("capi.hip", "capi", []),
@@ -59,8 +63,39 @@ def _compile(src: str, obj: str, defines) -> None:
         raise RuntimeError(f"hipcc failed for {os.path.basename(src)}:\n{res.stderr[-8000:]}")
 
 
+def _run(cmd, what: str) -> None:
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{what} failed:\n{res.stderr[-8000:]}")
+
+
+def _rocm() -> str:
+    return os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+
+
+def _compile_ops(obj: str) -> None:
+    import torch
+    from torch.utils import cpp_extension
+
+    inc = [*cpp_extension.include_paths(), os.path.join(_rocm(), "include"), sysconfig.get_paths()["include"]]
+    _run(["g++", "-std=c++17", "-O2", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{i}" for i in inc],
+          "-c", os.path.join(CSRC, "torch_ops.cpp"), "-o", obj], "g++ torch_ops.cpp")
+
+
+def _link_ops(obj: str) -> None:
+    from torch.utils import cpp_extension
+
+    out = os.path.join(LIBDIR, OPSNAME)
+    libs = [f"-L{p}" for p in (*cpp_extension.library_paths(), os.path.join(_rocm(), "lib"), LIBDIR)]
+    _run(["g++", "-shared", "-o", out + ".tmp", obj, *libs, f"-l:{LIBNAME}", "-ltorch", "-ltorch_cpu", "-ltorch_python",
+          "-lc10", "-lc10_hip", "-lamdhip64", "-Wl,-rpath,$ORIGIN"], "link of the torch ops")
+    os.replace(out + ".tmp", out)
+
+
 def build(verbose: bool = True) -> str:
-    """Compile every HIP source for gfx950 and link libmxf8.so; returns its path."""
+    """Compile every HIP source for gfx950 and link libmxf8.so (returns its path), then the
+    torch ops over it."""
     os.makedirs(LIBDIR, exist_ok=True)
     objdir = os.path.join(LIBDIR, "obj")
     os.makedirs(objdir, exist_ok=True)
@@ -70,6 +105,8 @@ def build(verbose: bool = True) -> str:
     workers = min(len(jobs), max(1, min(8, os.cpu_count() or 1)))
     with ThreadPoolExecutor(max_workers=workers) as ex:
         futs = [ex.submit(_compile, s, o, d) for s, o, d in jobs]
+        ops_obj = os.path.join(objdir, "torch_ops.o")
+        futs.append(ex.submit(_compile_ops, ops_obj))
         for f in futs:
             f.result()
     out = os.path.join(LIBDIR, LIBNAME)
@@ -79,8 +116,9 @@ def build(verbose: bool = True) -> str:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr[-8000:]}")
     os.replace(tmp, out)
+    _link_ops(ops_obj)
     if verbose:
-        print(f"[minimaxh3_amd] built {out}")
+        print(f"[minimaxh3_amd] built {out} and {OPSNAME}")
     return out
 
 

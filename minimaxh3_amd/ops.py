@@ -4,6 +4,10 @@ Registering the launches as ``torch.library.custom_op`` keeps the FP8 path opaqu
 torch.compile: the DiT blocks are compiled with ``fullgraph=False``
 (runtime/model_manager.py:127-141) and these ops trace as single nodes without graph
 breaks.  Outputs come from torch's caching allocator; launches go to the current stream.
+
+The ops of the hot path (quant_rows, adaln_quant_rows, gemm_rowwise, lora_down,
+attn_quant_kv, attn_fwd_q) run as native dispatcher kernels (csrc/torch_ops.cpp): their
+Python bodies only load those on the first GPU call.  The others call the C ABI from here.
 """
 from __future__ import annotations
 
@@ -24,6 +28,15 @@ def _prep(t: torch.Tensor, what: str) -> None:
     if not t.is_cuda:
         raise ValueError(f"{what}: expected a GPU tensor")
     N.require_gfx950(t.device)
+
+
+def _native(t: torch.Tensor, what: str):
+    """The native op ``mxf8::what``.  Runs when the dispatcher has no native kernel for the
+    call yet: refuses other devices, then registers the kernels, which take every later GPU
+    call before it reaches Python."""
+    _prep(t, what)
+    N.load_ops()
+    return getattr(torch.ops.mxf8, what).default
 
 
 def _on(t: torch.Tensor | None, device: torch.device, what: str) -> None:
@@ -77,17 +90,7 @@ def key_operands(key_mask: torch.Tensor | None, key_bias: torch.Tensor | None, B
 @torch.library.custom_op("mxf8::quant_rows", mutates_args=())
 def quant_rows(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """[M, K] bf16/fp16/fp32 -> (e4m3 [M, K], fp32 scale [M, 1]) (kernels/fp8_linear.py:27-42)."""
-    _prep(x, "quant_rows")
-    if x.stride(1) != 1 or x.stride(0) < x.shape[1]:
-        x = x.contiguous()
-    M, K = x.shape
-    x8 = torch.empty((M, K), dtype=E4M3, device=x.device)
-    scale = torch.empty((M, 1), dtype=torch.float32, device=x.device)
-    if M > 0:
-        with torch.cuda.device(x.device):
-            N.check(N.load().mxf8_quant_rows(x.data_ptr(), N.dtype_code(x.dtype), M, K, max(x.stride(0), K),
-                                             x8.data_ptr(), scale.data_ptr(), N.stream_of(x)), "quant_rows")
-    return x8, scale
+    return _native(x, "quant_rows")(x)
 
 
 @quant_rows.register_fake
@@ -106,33 +109,7 @@ def adaln_quant_rows(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor, 
     once (``eager=False``) or after every op like torch's eager bf16 ops (``eager=True``),
     and (x8, sa) = quant_rows(y).
     """
-    _prep(x, "adaln_quant_rows")
-    if x.ndim != 3 or shift.shape != (x.shape[0], x.shape[2]) or scale.shape != shift.shape:
-        raise ValueError("adaln_quant_rows: expected x [B, S, C] and shift, scale [B, C]")
-    if x.dtype != torch.bfloat16 or shift.dtype != torch.bfloat16 or scale.dtype != torch.bfloat16:
-        raise ValueError("adaln_quant_rows: bf16 tensors expected")
-    B, S, C = x.shape
-    x2 = x.reshape(B * S, C)
-    if x2.stride(1) != 1:
-        x2 = x2.contiguous()
-    # one row stride for both (expanded / strided operands are copied)
-    if shift.stride(1) != 1 or shift.stride(0) < C or shift.stride(0) % 8:
-        shift = shift.contiguous()
-    if scale.stride(1) != 1 or scale.stride(0) != shift.stride(0):
-        scale = scale.contiguous()
-        if scale.stride(0) != shift.stride(0):
-            shift = shift.contiguous()
-    M = B * S
-    x8 = torch.empty((M, C), dtype=E4M3, device=x.device)
-    sa = torch.empty((M, 1), dtype=torch.float32, device=x.device)
-    y = torch.empty((M, C) if want_y else (0,), dtype=torch.bfloat16, device=x.device)
-    if M > 0:
-        with torch.cuda.device(x.device):
-            N.check(N.load().mxf8_adaln_quant_rows(
-                x2.data_ptr(), M, C, x2.stride(0), S, shift.data_ptr(), scale.data_ptr(), shift.stride(0),
-                float(eps), int(bool(eager)), x8.data_ptr(), sa.data_ptr(), y.data_ptr() if want_y else None,
-                N.stream_of(x)), "adaln_quant_rows")
-    return x8, sa, y
+    return _native(x, "adaln_quant_rows")(x, shift, scale, eps, eager, want_y)
 
 
 @adaln_quant_rows.register_fake
@@ -147,36 +124,7 @@ def gemm_rowwise(a8: torch.Tensor, w8: torch.Tensor, sa: torch.Tensor, sw: torch
                  bias: torch.Tensor | None, act: int, lora_t: torch.Tensor | None,
                  lora_b: torch.Tensor | None, lora_scale: float) -> torch.Tensor:
     """bf16(a8 w8^T * sa * sw + bias) (+ LoRA) (+ GELU-tanh), bf16 [M, N]."""
-    _prep(a8, "gemm_rowwise")
-    M, K = a8.shape
-    Nn = w8.shape[0]
-    dev = a8.device
-    if a8.dtype != E4M3 or w8.dtype != E4M3 or w8.dim() != 2 or w8.shape[1] != K:
-        raise ValueError(f"gemm_rowwise: e4m3 a8 [M, K] and w8 [N, K] expected, got {a8.dtype} {tuple(a8.shape)} "
-                         f"and {w8.dtype} {tuple(w8.shape)}")
-    if not (a8.is_contiguous() and w8.is_contiguous()):
-        raise ValueError("gemm_rowwise: a8 and w8 must be contiguous")
-    if sa.dtype != torch.float32 or sa.numel() != M or sw.dtype != torch.float32 or sw.numel() != Nn:
-        raise ValueError(f"gemm_rowwise: fp32 scales of {M} rows and {Nn} channels expected")
-    if not (sa.is_contiguous() and sw.is_contiguous()):
-        raise ValueError("gemm_rowwise: scales must be contiguous")
-    if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != Nn or not bias.is_contiguous()):
-        raise ValueError(f"gemm_rowwise: bias must be {Nn} contiguous bf16 values")
-    if lora_t is not None and (lora_b is None or lora_t.shape[0] != M or lora_b.shape != (Nn, lora_t.shape[1])
-                               or not lora_t.is_contiguous() or not lora_b.is_contiguous()):
-        raise ValueError("gemm_rowwise: LoRA operands t [M, r] and B [N, r] (contiguous bf16) expected")
-    for t, name in ((w8, "w8"), (sa, "sa"), (sw, "sw"), (bias, "bias"), (lora_t, "lora_t"), (lora_b, "lora_b")):
-        _on(t, dev, f"gemm_rowwise: {name}")
-    out = torch.empty((M, Nn), dtype=torch.bfloat16, device=a8.device)
-    if M == 0 or Nn == 0:
-        return out
-    r = 0 if lora_t is None else lora_t.shape[1]
-    with torch.cuda.device(a8.device):
-        N.check(N.load().mxf8_gemm_rowwise(
-            a8.data_ptr(), w8.data_ptr(), sa.data_ptr(), sw.data_ptr(), N.ptr(bias), int(act),
-            N.ptr(lora_t), N.ptr(lora_b), r, float(lora_scale), out.data_ptr(), M, Nn, K, Nn,
-            N.stream_of(a8)), "gemm_rowwise")
-    return out
+    return _native(a8, "gemm_rowwise")(a8, w8, sa, sw, bias, act, lora_t, lora_b, lora_scale)
 
 
 @gemm_rowwise.register_fake
@@ -233,18 +181,7 @@ def _(a8, w8, sa, sw, bias, seq_len, k_col0, v_col0, cols):
 @torch.library.custom_op("mxf8::lora_down", mutates_args=())
 def lora_down(x: torch.Tensor, a: torch.Tensor) -> torch.Tensor:
     """t = bf16(x A^T): x [M, K] bf16, A [r, K] bf16 -> [M, r] bf16 (kernels/fp8_linear.py:53)."""
-    _prep(x, "lora_down")
-    if x.stride(1) != 1:
-        x = x.contiguous()
-    a = a.contiguous()
-    M, K = x.shape
-    r = a.shape[0]
-    t = torch.empty((M, r), dtype=torch.bfloat16, device=x.device)
-    if M > 0:
-        with torch.cuda.device(x.device):
-            N.check(N.load().mxf8_lora_down(x.data_ptr(), x.stride(0), a.data_ptr(), t.data_ptr(), M, K, r,
-                                            N.stream_of(x)), "lora_down")
-    return t
+    return _native(x, "lora_down")(x, a)
 
 
 @lora_down.register_fake
@@ -352,24 +289,7 @@ def attn_quant_kv(k: torch.Tensor, v: torch.Tensor) -> tuple[torch.Tensor, torch
     """K and V quantized together (fp8_attention.py:338-369): (K8 [B,H,Skp,D], sk [B,H,nk],
     V8T [B,H,D,Skp], sv [B,H,D], key mean [B,H,D] fp32) -- the outputs of attn_kmean +
     attn_quant_k + attn_quant_v in three launches."""
-    _prep(k, "attn_quant_kv")
-    if k.shape != v.shape or k.dtype != v.dtype or k.device != v.device:
-        raise ValueError("attn_quant_kv: k and v must have one shape, dtype and device")
-    B, H, S, D = k.shape
-    nk = _cdiv(S, 128)
-    k8 = torch.empty((B, H, nk * 128, D), dtype=E4M3, device=k.device)
-    sk = torch.empty((B, H, nk), dtype=torch.float32, device=k.device)
-    v8t = torch.empty((B, H, D, nk * 128), dtype=E4M3, device=k.device)
-    sv = torch.empty((B, H, D), dtype=torch.float32, device=k.device)
-    mean = torch.empty((B, H, D), dtype=torch.float32, device=k.device)
-    ws = torch.empty(max(int(N.load().mxf8_attn_kv_workspace_bytes(B, H, S, D)), 16), dtype=torch.uint8,
-                     device=k.device)
-    with torch.cuda.device(k.device):
-        N.check(N.load().mxf8_attn_quant_kv(
-            k.data_ptr(), N.strides4(k), v.data_ptr(), N.strides4(v), N.dtype_code(k.dtype), B, H, S, D,
-            k8.data_ptr(), sk.data_ptr(), v8t.data_ptr(), sv.data_ptr(), mean.data_ptr(), ws.data_ptr(),
-            N.stream_of(k)), "attn_quant_kv")
-    return k8, sk, v8t, sv, mean
+    return _native(k, "attn_quant_kv")(k, v)
 
 
 @attn_quant_kv.register_fake
@@ -481,24 +401,7 @@ def attn_fwd_q(q: torch.Tensor, c: float, k8: torch.Tensor, v8t: torch.Tensor, s
     """attn_quant_q + attn_fwd in one launch (fp8_attention.py:321-336 and 380-402): each
     128-row Q block is quantized inside the launch; same output bit for bit.  kv_mode as
     attn_fwd."""
-    _prep(q, "attn_fwd_q")
-    if not attn_fwd_q_supported(q):
-        raise ValueError("attn_fwd_q: q must be bf16/fp16 with unit channel stride, other strides multiples of 8 "
-                         "and 16-byte alignment")
-    if q.data_ptr() % 16:
-        # a view that starts off a 16-byte boundary: the two launches give the same bits
-        q8, sq = attn_quant_q(q, c)
-        return attn_fwd(q8, k8, v8t, sq, sk, sv, key_mask, key_bias, repair_tau, q, Sk, kv_mode)
-    B, H, Sq, D = q.shape
-    _check_kv_codes(k8, v8t, sk, sv, B, H, Sk, D, q.device, "attn_fwd_q")
-    out = torch.empty_like(q)
-    km, kb = key_operands(key_mask, key_bias, B, Sk, q.device)
-    with torch.cuda.device(q.device):
-        N.check(N.load().mxf8_attn_fwd_q(
-            q.data_ptr(), N.strides4(q), float(c), k8.data_ptr(), v8t.data_ptr(), sk.data_ptr(), sv.data_ptr(),
-            N.ptr(km), N.ptr(kb), float(repair_tau), None, out.data_ptr(), N.dtype_code(out.dtype), N.strides4(out),
-            B, H, Sq, Sk, D, int(kv_mode), N.stream_of(q)), "attn_fwd_q")
-    return out
+    return _native(q, "attn_fwd_q")(q, c, k8, v8t, sk, sv, key_mask, key_bias, repair_tau, Sk, kv_mode)
 
 
 @attn_fwd_q.register_fake
