@@ -357,10 +357,11 @@ __device__ __forceinline__ void load8(const void* base, const Strides4& st, int6
 
 // Q (IS_K = false) and K (IS_K = true) quantizer of one (128-row block blk, b*H + h) tile
 // by a 256-thread block (nblk blocks per head; red: 4 floats of LDS).  Thread t handles
-// the 8-wide d-chunk (t % CPR) of rows (t / CPR) + RPP * p.
-template <int DT, int D, bool IS_K, bool VEC>
+// the 8-wide d-chunk (t % CPR) of rows (t / CPR) + RPP * p.  mean_of() gives the head's key
+// mean (D values); it is called once the tile's loads are in flight.
+template <int DT, int D, bool IS_K, bool VEC, class MeanFn>
 __device__ __forceinline__ void quant_qk_tile(const void* __restrict__ src, const Strides4& st, int64_t H, int64_t S,
-                                              int64_t Sp, float c, const float* __restrict__ mean,
+                                              int64_t Sp, float c, MeanFn mean_of,
                                               uint8_t* __restrict__ out8, float* __restrict__ scale_out, int64_t blk,
                                               int64_t bh, int64_t nblk, float* red) {
   constexpr int CPR = D / 8;      // chunks per row
@@ -370,11 +371,6 @@ __device__ __forceinline__ void quant_qk_tile(const void* __restrict__ src, cons
   const void* base = static_cast<const char*>(src) + (b * st.b + h * st.h) * (int64_t)sizeof(typename Elem<DT>::T);
   const int cc = threadIdx.x % CPR;
   const int rl = threadIdx.x / CPR;
-  float mu[8];
-  if constexpr (IS_K) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) mu[i] = mean[bh * D + cc * 8 + i];
-  }
   float f[NP][8];
   float amax = 0.0f;
   uint4 raw[VEC ? NP : 1];
@@ -385,6 +381,12 @@ __device__ __forceinline__ void quant_qk_tile(const void* __restrict__ src, cons
       const int64_t s = blk * 128 + rl + RPP * p;
       raw[p] = s < S ? raw8<DT>(base, st, s, cc * 8) : make_uint4(0, 0, 0, 0);
     }
+  }
+  float mu[8];
+  if constexpr (IS_K) {
+    const float* const mean = mean_of();
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mu[i] = mean[cc * 8 + i];
   }
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
@@ -429,8 +431,8 @@ __global__ __launch_bounds__(256) void attn_quant_qk_kernel(const void* __restri
                                                             uint8_t* __restrict__ out8,
                                                             float* __restrict__ scale_out) {
   __shared__ float red[4];
-  quant_qk_tile<DT, D, IS_K, VEC>(src, st, H, S, Sp, c, mean, out8, scale_out, blockIdx.x, blockIdx.y, gridDim.x,
-                                  red);
+  quant_qk_tile<DT, D, IS_K, VEC>(src, st, H, S, Sp, c, [&] { return mean + (int64_t)blockIdx.y * D; }, out8,
+                                  scale_out, blockIdx.x, blockIdx.y, gridDim.x, red);
 }
 
 // Partial column reductions over a chunk of rows: SUM (key mean) or ABSMAX (V scale).
@@ -541,7 +543,8 @@ __global__ __launch_bounds__(256) void attn_colfold_kernel(const float* __restri
 // V quantizer of one (128-key tile blk, b*H + h), transposed store: the block quantizes a
 // 128-key x D tile with the per-channel scales sv and writes it transposed through LDS so
 // that every v8t row segment is a full 128 bytes.  Thread t handles d-chunk (t % CPR) of
-// the 4 consecutive keys 4 * (t / CPR + KQP * p) + 0..3.
+// the 4 consecutive keys 4 * (t / CPR + KQP * p) + 0..3.  scale_of() gives the head's D channel
+// scales; it is called once the tile's loads are in flight.
 template <int D>
 struct QuantVLds {
   static constexpr int STRIDE = 128 + 4;  // LDS row stride of the transposed tile
@@ -550,9 +553,9 @@ struct QuantVLds {
   float s_r[D];
 };
 
-template <int DT, int D, bool VEC>
+template <int DT, int D, bool VEC, class ScaleFn>
 __device__ __forceinline__ void quant_v_tile(const void* __restrict__ src, const Strides4& st, int64_t H, int64_t S,
-                                             int64_t Sp, const float* __restrict__ sv, uint8_t* __restrict__ v8t,
+                                             int64_t Sp, ScaleFn scale_of, uint8_t* __restrict__ v8t,
                                              int64_t blk, int64_t bh, QuantVLds<D>& L) {
   constexpr int CPR = D / 8;
   constexpr int KQP = 256 / CPR;  // key quads per pass
@@ -562,14 +565,25 @@ __device__ __forceinline__ void quant_v_tile(const void* __restrict__ src, const
   float* const s_sv = L.s_sv;
   float* const s_r = L.s_r;
   const int64_t b = bh / H, h = bh % H;
+  const void* base = static_cast<const char*>(src) + (b * st.b + h * st.h) * (int64_t)sizeof(typename Elem<DT>::T);
+  const int cc = threadIdx.x % CPR;
+  uint4 raw[VEC ? NP : 1][VEC ? 4 : 1];
+  if constexpr (VEC) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t s = blk * 128 + (threadIdx.x / CPR + KQP * p) * 4 + j;
+        raw[p][j] = s < S ? raw8<DT>(base, st, s, cc * 8) : make_uint4(0, 0, 0, 0);
+      }
+  }
+  const float* const sv = scale_of();
   if (threadIdx.x < D) {
-    const float s = sv[bh * D + threadIdx.x];
+    const float s = sv[threadIdx.x];
     s_sv[threadIdx.x] = s;
     s_r[threadIdx.x] = __fdiv_rn(1.0f, s);
   }
   __syncthreads();
-  const void* base = static_cast<const char*>(src) + (b * st.b + h * st.h) * (int64_t)sizeof(typename Elem<DT>::T);
-  const int cc = threadIdx.x % CPR;
   float scl[8], rcp[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -580,21 +594,13 @@ __device__ __forceinline__ void quant_v_tile(const void* __restrict__ src, const
   for (int p = 0; p < NP; ++p) {
     const int kq = threadIdx.x / CPR + KQP * p;
     uint32_t col[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // col[i]: 4 key bytes of channel cc*8+i
-    uint4 raw[VEC ? 4 : 1];
-    if constexpr (VEC) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t s = blk * 128 + kq * 4 + j;
-        raw[j] = s < S ? raw8<DT>(base, st, s, cc * 8) : make_uint4(0, 0, 0, 0);
-      }
-    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int64_t s = blk * 128 + kq * 4 + j;
       float f[8];
       if (s < S) {
         if constexpr (VEC)
-          cvt8<DT>(raw[j], f);
+          cvt8<DT>(raw[p][j], f);
         else
           load8<DT, VEC>(base, st, s, cc * 8, f);
       } else {
@@ -629,13 +635,15 @@ __global__ __launch_bounds__(256) void attn_quant_v_kernel(const void* __restric
                                                            int64_t S, int64_t Sp, const float* __restrict__ sv,
                                                            uint8_t* __restrict__ v8t) {
   __shared__ QuantVLds<D> L;
-  quant_v_tile<DT, D, VEC>(src, st, H, S, Sp, sv, v8t, blockIdx.x, blockIdx.y, L);
+  quant_v_tile<DT, D, VEC>(src, st, H, S, Sp, [&] { return sv + (int64_t)blockIdx.y * D; }, v8t, blockIdx.x,
+                           blockIdx.y, L);
 }
 
 // ---------------------------------------------------------------------------------------
 // K and V of one attention together (kernels/fp8_attention.py:338-369): one pass over both
 // for the statistics that need the whole sequence (the key mean, the per-channel V amax),
-// one fold of both, then one launch that quantizes a 128-key tile of K and of V per block.
+// one fold of both (for few keys inside the quantizing blocks, kv_fold_in_quant), then one
+// launch that quantizes a 128-key tile of K or of V per block.
 // The second read of K and V follows the first closely, so it is mostly served by the
 // MALL; in the fused QKV layout ([B, S, 2, H, D]) the two reads of a key's K and V rows
 // are adjacent.
@@ -728,19 +736,53 @@ __global__ __launch_bounds__(256) void attn_kv_fold_kernel(const float* __restri
   }
 }
 
-// K tile and V tile of the same 128 keys (grid (B*H, Skp/128)).
-template <int DT, int D, bool VECK, bool VECV>
+// Quantizes the K tile (even blockIdx.x) or the V tile (odd) of 128 keys of one head (grid
+// (2 B*H, Skp/128)): heads fastest, so the blocks that run together read the same keys' rows,
+// and K and V in blocks of their own, which halves the chain of loads, statistics, codes and
+// stores that a launch of few tiles consists of.
+//
+// FOLD: the block folds its head's statistic from the partial slabs itself (every block of a
+// head the same way, attn_kv_fold_kernel's order and so its bits), and the head's first block
+// writes it out: no fold launch.
+template <int DT, int D, bool VECK, bool VECV, bool FOLD>
 __global__ __launch_bounds__(256) void attn_quant_kv_kernel(const void* __restrict__ k, Strides4 stk,
                                                             const void* __restrict__ v, Strides4 stv, int64_t H,
-                                                            int64_t S, int64_t Sp, const float* __restrict__ mean,
-                                                            const float* __restrict__ sv, uint8_t* __restrict__ k8,
-                                                            float* __restrict__ sk, uint8_t* __restrict__ v8t) {
-  __shared__ float red[4];
+                                                            int64_t S, int64_t Sp, const float* __restrict__ part,
+                                                            int nch, float* __restrict__ mean, float* __restrict__ sv,
+                                                            uint8_t* __restrict__ k8, float* __restrict__ sk,
+                                                            uint8_t* __restrict__ v8t) {
+  __shared__ float red[FOLD ? 256 : 4];
+  __shared__ float stat[FOLD ? D : 1];
   __shared__ QuantVLds<D> L;
-  // heads fastest: blocks that run together read the same keys' rows
-  const int64_t bh = blockIdx.x, blk = blockIdx.y, nb = gridDim.y;
-  quant_qk_tile<DT, D, true, VECK>(k, stk, H, S, Sp, 0.0f, mean, k8, sk, blk, bh, nb, red);
-  quant_v_tile<DT, D, VECV>(v, stv, H, S, Sp, sv, v8t, blk, bh, L);
+  const int64_t bh = blockIdx.x >> 1, blk = blockIdx.y, nb = gridDim.y, BH = gridDim.x >> 1;
+  if (blockIdx.x & 1) {
+    quant_v_tile<DT, D, VECV>(v, stv, H, S, Sp, [&]() -> const float* {
+      if constexpr (FOLD) {
+        const float amax = colfold<D, true>(part + BH * nch * D, nch, bh, red);
+        if (threadIdx.x < D) {
+          stat[threadIdx.x] = e4m3_scale(amax);
+          if (blk == 0) sv[bh * D + threadIdx.x] = stat[threadIdx.x];
+        }
+        return stat;  // (a thread reads only what it wrote)
+      } else {
+        return sv + bh * D;
+      }
+    }, v8t, blk, bh, L);
+  } else {
+    quant_qk_tile<DT, D, true, VECK>(k, stk, H, S, Sp, 0.0f, [&]() -> const float* {
+      if constexpr (FOLD) {
+        const float sum = colfold<D, false>(part, nch, bh, red);
+        if (threadIdx.x < D) {
+          stat[threadIdx.x] = __fdiv_rn(sum, (float)S);
+          if (blk == 0) mean[bh * D + threadIdx.x] = stat[threadIdx.x];
+        }
+        __syncthreads();
+        return stat;
+      } else {
+        return mean + bh * D;
+      }
+    }, k8, sk, blk, bh, nb, red);
+  }
 }
 
 // Fold of the K/V column statistics that the QKV projection's epilogue emits
@@ -1028,6 +1070,14 @@ extern "C" int64_t mxf8_attn_kv_workspace_bytes(int64_t B, int64_t H, int64_t S,
   return (2 * (int64_t)colreduce_chunks(BH, S) + 1) * BH * D * (int64_t)sizeof(float);
 }
 
+// Whether the quantizing blocks fold the statistics themselves: every one of the B*H*nb pairs
+// reads its head's slabs again (2 nch D floats from the L2), against one fold launch.  MI355X,
+// 24 heads, D = 128, all launches, folded there / in a launch of their own: 1024 keys (3 MB of
+// re-reads) 12.5 / 14.8 us, 4673 keys (58 MB) 31.3 / 33.5, 20280 keys (250 MB) 115.5 / 107.7.
+static bool kv_fold_in_quant(int64_t BH, int64_t nb, int nch, int64_t D) {
+  return BH * nb * nch * 2 * D * (int64_t)sizeof(float) <= ((int64_t)64 << 20);
+}
+
 template <int DT, int D>
 static void launch_kv(const void* k, const Strides4& stk, bool veck, const void* v, const Strides4& stv, bool vecv,
                       int64_t H, int64_t S, int64_t BH, int nch, float* part, float* mean, float* sv, uint8_t* k8,
@@ -1035,13 +1085,19 @@ static void launch_kv(const void* k, const Strides4& stk, bool veck, const void*
   const int64_t rpc = cdiv(S, nch);
   const dim3 rgrid((unsigned)BH, (unsigned)nch);
   const int64_t nb = cdiv(S, 128);
-  const dim3 qgrid((unsigned)BH, (unsigned)nb);
+  const dim3 qgrid((unsigned)(2 * BH), (unsigned)nb);
+  const bool fold = kv_fold_in_quant(BH, nb, nch, D);
 #define MXF8_KV_CASE(VK, VV)                                                                                     \
   if (veck == VK && vecv == VV) {                                                                                \
     attn_kv_colreduce_kernel<DT, D, VK, VV><<<rgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, rpc, part);         \
+    if (fold) {                                                                                                  \
+      attn_quant_kv_kernel<DT, D, VK, VV, true><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128, part, \
+                                                                            nch, mean, sv, k8, sk, v8t);         \
+      return;                                                                                                    \
+    }                                                                                                            \
     attn_kv_fold_kernel<D><<<dim3((unsigned)BH), 256, 0, stream>>>(part, nch, S, mean, sv);                       \
-    attn_quant_kv_kernel<DT, D, VK, VV><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128, mean, sv, k8, \
-                                                                    sk, v8t);                                    \
+    attn_quant_kv_kernel<DT, D, VK, VV, false><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128, nullptr, \
+                                                                           0, mean, sv, k8, sk, v8t);            \
     return;                                                                                                      \
   }
   MXF8_KV_CASE(true, true)
@@ -1054,14 +1110,14 @@ static void launch_kv(const void* k, const Strides4& stk, bool veck, const void*
 // The quantizing pass of the K/V pair alone (the key mean and V scales given).
 template <int DT, int D>
 static void launch_quant_kv_only(const void* k, const Strides4& stk, bool veck, const void* v, const Strides4& stv,
-                                 bool vecv, int64_t H, int64_t S, int64_t BH, const float* mean, const float* sv,
+                                 bool vecv, int64_t H, int64_t S, int64_t BH, float* mean, float* sv,
                                  uint8_t* k8, float* sk, uint8_t* v8t, hipStream_t stream) {
   const int64_t nb = cdiv(S, 128);
-  const dim3 qgrid((unsigned)BH, (unsigned)nb);
+  const dim3 qgrid((unsigned)(2 * BH), (unsigned)nb);
 #define MXF8_KVQ_CASE(VK, VV)                                                                                    \
   if (veck == VK && vecv == VV) {                                                                                \
-    attn_quant_kv_kernel<DT, D, VK, VV><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128, mean, sv, k8, \
-                                                                    sk, v8t);                                    \
+    attn_quant_kv_kernel<DT, D, VK, VV, false><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128, nullptr, \
+                                                                           0, mean, sv, k8, sk, v8t);            \
     return;                                                                                                      \
   }
   MXF8_KVQ_CASE(true, true)
