@@ -83,17 +83,17 @@ __global__ __launch_bounds__(C::THREADS) void gemm_ring_kernel(
   // The epilogue's operands are read first and handed over through LDS while the first
   // stages are in flight (indices past M or N read the last element; those outputs are not
   // stored).
+  // (Unconditional loads from selected addresses: a load under a condition would be waited
+  // for where the condition ends, before the first copy is issued.)
   constexpr int NEP = (C::EP + C::THREADS - 1) / C::THREADS;
   float epv[NEP];
+  uint16_t epb[NEP];
 #pragma unroll
   for (int e = 0; e < NEP; ++e) {
-    const int i = min(threadIdx.x + e * C::THREADS, C::EP - 1);
-    if (i < C::BN)
-      epv[e] = sw[min(n0 + i, N - 1)];
-    else if (i < 2 * C::BN)
-      epv[e] = bias ? bf16_bits_to_f32(bias[min(n0 + i - C::BN, N - 1)]) : 0.0f;
-    else
-      epv[e] = sa[min(m0 + i - 2 * C::BN, M - 1)];
+    const int i = min((int)threadIdx.x + e * C::THREADS, C::EP - 1);
+    const int ch = min(n0 + (i < C::BN ? i : i < 2 * C::BN ? i - C::BN : 0), N - 1);
+    epv[e] = *(i < 2 * C::BN ? sw + ch : sa + min(m0 + i - 2 * C::BN, M - 1));
+    epb[e] = *(bias ? bias + ch : reinterpret_cast<const uint16_t*>(sw));
   }
 #pragma unroll
   for (int s = 0; s < NS; ++s)
@@ -101,7 +101,8 @@ __global__ __launch_bounds__(C::THREADS) void gemm_ring_kernel(
 #pragma unroll
   for (int e = 0; e < NEP; ++e) {
     const int i = threadIdx.x + e * C::THREADS;
-    if (i < C::EP) ep[i] = epv[e];
+    if (i < C::EP)
+      ep[i] = i < C::BN || i >= 2 * C::BN ? epv[e] : bias ? bf16_bits_to_f32(epb[e]) : 0.0f;
   }
 
   v16f acc[TN][TM];
@@ -223,12 +224,12 @@ typedef GemmRing<128, 128, 2, 4, 4, 1> GemmRing128x128; // 128 KB: one
 
 // Estimated time (us) of `tiles` workgroups, `per_cu` of them resident on a CU, over ns
 // 128-byte stages of K: a start-up cost, then per round t1 per stage with one workgroup on a
-// CU or t2 with two, and the LoRA branch's `lora`.
+// CU or t2 with two, and the LoRA branch's `lora` per workgroup on a CU.
 inline float gemm_time(int64_t tiles, int cus, int per_cu, int64_t ns, float start, float t1, float t2, float lora) {
   if (per_cu == 1) return start + (float)cdiv(tiles, cus) * (t1 * (float)ns + lora);
   const int64_t full = tiles / (2 * cus), rem = tiles - full * 2 * cus;
-  return start + (float)full * (t2 * (float)ns + lora) +
-         (rem == 0 ? 0.0f : (rem <= cus ? t1 : t2) * (float)ns + lora);
+  return start + (float)full * (t2 * (float)ns + 2.0f * lora) +
+         (rem == 0 ? 0.0f : rem <= cus ? t1 * (float)ns + lora : t2 * (float)ns + 2.0f * lora);
 }
 
 // The ring tile for an M x N x K product (0-3 in the order above), or -1 where
@@ -240,7 +241,7 @@ inline float gemm_time(int64_t tiles, int cus, int per_cu, int64_t ns, float sta
 // where M <= 1280 leaves CUs without a 128 x 128 tile.  Past that the larger tile reads fewer
 // operand bytes from the L2s and wins (2048 x 3072 x 3072: 22.6 us against 29.2 with 128 x 64).
 // A LoRA of rank r (0 without) costs the ring tiles 0.5-3.7 us per 64 ranks, read from global
-// memory in the epilogue, and the 128 x 128 tiles 1.2 us from LDS (r <= 128) or 4 (1024 x 3072
+// memory in the epilogue, and the 128 x 128 tiles 1 us from LDS (r <= 128) or 2.4 (1024 x 3072
 // x 3072, rank 128: 22.4 us there against 24.0).
 inline int gemm_ring_pick(int64_t M, int64_t N, int64_t K, int64_t r, int cus) {
   const int64_t ns = cdiv(K, GEMM_BK);
@@ -252,7 +253,7 @@ inline int gemm_ring_pick(int64_t M, int64_t N, int64_t K, int64_t r, int cus) {
                       gemm_time(tiles(128, 128), cus, 1, ns, 2.1f, 0.66f, 0.0f, 3.7f * l)};
   // (two stage buffers; long-K panels share the L2s less)
   const float base = gemm_time(tiles(128, 128), cus, 2, ns, 2.25f, K < 8192 ? 0.78f : 1.0f, K < 8192 ? 1.16f : 1.12f,
-                               (r <= 128 ? 1.2f : 4.0f) * l);
+                               (r <= 128 ? 1.0f : 2.4f) * l);
   int best = 0;
   for (int i = 1; i < 4; ++i)
     if (t[i] < t[best]) best = i;
