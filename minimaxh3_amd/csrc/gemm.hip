@@ -964,29 +964,33 @@ extern "C" int mxf8_gemm_rowwise(const uint8_t* a8, const uint8_t* w8, const flo
   const uint16_t* lt = static_cast<const uint16_t*>(lora_t);
   const uint16_t* lb = static_cast<const uint16_t*>(lora_b);
   uint16_t* o16 = static_cast<uint16_t*>(out);
-  // 256x256 tiles when they fill the chip; below that the ring kernel where it is faster,
-  // 128x128 otherwise.
-  const int64_t big_tiles = cdiv(M, 256) * cdiv(N, 256);
   const int cus = device_cus();
-  const int ring = big_tiles >= 2 * 256 || cus <= 0 ? -1 : gemm_ring_pick(M, N, K, lora ? r : 0, cus);
-  if (ring == 0)
-    launch_gemm_ring<GemmRing32x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
-                                    ld_out, stream);
-  else if (ring == 1)
-    launch_gemm_ring<GemmRing64x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
-                                    ld_out, stream);
-  else if (ring == 2)
-    launch_gemm_ring<GemmRing128x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
-                                     ld_out, stream);
-  else if (ring == 3)
-    launch_gemm_ring<GemmRing128x128>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
-                                      ld_out, stream);
-  else if (big_tiles >= 2 * 256)
-    gemm_dispatch_tile<GemmBig>(act, lm, ktail, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
-                                ld_out, stream);
-  else
-    gemm_dispatch_tile<GemmSmall>(act, lm, ktail, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
+  if (cus <= 0) return set_error(MXF8_ELAUNCH, "gemm_rowwise: the device's compute-unit count is unavailable");
+  switch (gemm_pick(M, N, K, lora ? r : 0, cus)) {
+    case 0:
+      launch_gemm_ring<GemmRing32x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK, ld_out,
+                                      stream);
+      break;
+    case 1:
+      launch_gemm_ring<GemmRing64x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK, ld_out,
+                                      stream);
+      break;
+    case 2:
+      launch_gemm_ring<GemmRing128x64>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK, ld_out,
+                                       stream);
+      break;
+    case 3:
+      launch_gemm_ring<GemmRing128x128>(act, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK, ld_out,
+                                        stream);
+      break;
+    case GEMM_TILE_256:
+      gemm_dispatch_tile<GemmBig>(act, lm, ktail, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
                                   ld_out, stream);
+      break;
+    default:
+      gemm_dispatch_tile<GemmSmall>(act, lm, ktail, a8, w8, sa, sw, b16, lt, lb, (int)r, lora_scale, o16, iM, iN, iK,
+                                    ld_out, stream);
+  }
   return check_launch("gemm_rowwise");
 }
 
@@ -1032,8 +1036,10 @@ extern "C" int mxf8_gemm_rowwise_kv_stats(const uint8_t* a8, const uint8_t* w8, 
   const uint16_t* b16 = static_cast<const uint16_t*>(bias);
   uint16_t* o16 = static_cast<uint16_t*>(out);
   const bool ktail = (K % GEMM_BK) != 0;
-  // the tile choice of mxf8_gemm_rowwise, so the output is that entry point's bit for bit
-  const bool big = cdiv(M, 256) * cdiv(N, 256) >= 2 * 256;
+  // (the output is mxf8_gemm_rowwise's bit for bit whatever tile either takes)
+  const int cus = device_cus();
+  if (cus <= 0) return set_error(MXF8_ELAUNCH, "%s: the device's compute-unit count is unavailable", what);
+  const bool big = gemm_use_big(M, N, K, 0, cus, gemm_time_small(M, N, K, 0, cus));
 #define MXF8_KVS_LAUNCH(Cfg, T)                                                                                    \
   launch_gemm<Cfg, MXF8_ACT_NONE, LORA_NONE, T, true>(a8, w8, sa, sw, b16, nullptr, nullptr, 0, 0.0f, o16, iM, iN, \
                                                       iK, ld_out, stream, kvs)
