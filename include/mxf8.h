@@ -183,7 +183,8 @@ int64_t mxf8_attn_kv_workspace_bytes(int64_t B, int64_t H, int64_t S, int64_t D)
  * _quantize_k_kernel (80-119, launch 339-354) and _quantize_v_kernel (122-170, launch
  * 356-369) of one attention call: the same outputs as mxf8_attn_kmean + mxf8_attn_quant_k +
  * mxf8_attn_quant_v, in three launches (one pass over K and V for the key mean and the
- * per-channel V amax, one fold of both, one pass that quantizes K and V).
+ * per-channel V amax, one fold of both, one pass that quantizes K and V; for few
+ * keys the last folds as well).
  *   k, v [B, H, S, D] of `dtype` with element strides k_strides[4], v_strides[4]
  *   k8 [B, H, Skp, D], sk [B, H, ceil(S/128)], v8t [B, H, D, Skp], sv [B, H, D] (written)
  *   mean [B, H, D] fp32 key mean (written when not NULL; kept in `workspace` otherwise)

@@ -9,9 +9,9 @@
 // HBM).  Here the tile is small enough to give every CU one, the ring keeps NS - 1 stages of
 // copies in flight, and a stage's fragments are read from LDS while the previous stage's
 // products run, so a stage costs 0.25-0.7 us (by tile size, gemm_pick).  MI355X, weights
-// from HBM, before -> after: 1 x 3072 x 3072 16.7 -> 8.0 us, 512 x 3072 x 3072 18.9 -> 11.3,
-// 1 x 9216 x 3072 23.2 -> 9.6, 256 x 9216 x 3072 26.8 -> 19.9, 1 x 3072 x 12288 82 -> 23.8,
-// 1024 x 3072 x 12288 104 -> 65 us.  Splitting K over workgroups would shorten the chain
+// from HBM, before -> after: 1 x 3072 x 3072 16.7 -> 8.0 us, 512 x 3072 x 3072 18.9 -> 11.7,
+// 1 x 9216 x 3072 23.2 -> 10.3, 256 x 9216 x 3072 26.6 -> 19.9, 1 x 3072 x 12288 83.6 -> 23.6,
+// 1024 x 3072 x 12288 103.7 -> 64.7 us.  Splitting K over workgroups would shorten the chain
 // further, but would sum the products in another order.
 #pragma once
 

@@ -1128,7 +1128,8 @@ static void launch_quant_kv_only(const void* k, const Strides4& stk, bool veck, 
 }
 
 // K and V quantized together: the key mean, the K quantizer, the per-channel V scale and
-// the transposed V quantizer (kernels/fp8_attention.py:338-369) in three launches.
+// the transposed V quantizer (kernels/fp8_attention.py:338-369) in three launches, two
+// where kv_fold_in_quant puts the fold into the last.
 static int attn_quant_kv_impl(const char* what, const void* k, const int64_t k_strides[4], const void* v,
                               const int64_t v_strides[4], int dtype, int64_t B, int64_t H, int64_t S, int64_t D,
                               uint8_t* k8, float* sk, uint8_t* v8t, float* sv, float* mean, float* part, int nch,

@@ -288,7 +288,7 @@ def attn_quant_kv(k: torch.Tensor, v: torch.Tensor) -> tuple[torch.Tensor, torch
                                                             torch.Tensor]:
     """K and V quantized together (fp8_attention.py:338-369): (K8 [B,H,Skp,D], sk [B,H,nk],
     V8T [B,H,D,Skp], sv [B,H,D], key mean [B,H,D] fp32) -- the outputs of attn_kmean +
-    attn_quant_k + attn_quant_v in three launches."""
+    attn_quant_k + attn_quant_v in two or three launches."""
     return _native(k, "attn_quant_kv")(k, v)
 
 
