@@ -1036,10 +1036,11 @@ extern "C" int mxf8_gemm_rowwise_kv_stats(const uint8_t* a8, const uint8_t* w8, 
   const uint16_t* b16 = static_cast<const uint16_t*>(bias);
   uint16_t* o16 = static_cast<uint16_t*>(out);
   const bool ktail = (K % GEMM_BK) != 0;
-  // (the output is mxf8_gemm_rowwise's bit for bit whatever tile either takes)
-  const int cus = device_cus();
-  if (cus <= 0) return set_error(MXF8_ELAUNCH, "%s: the device's compute-unit count is unavailable", what);
-  const bool big = gemm_use_big(M, N, K, 0, cus, gemm_time_small(M, N, K, 0, cus));
+  // The output is mxf8_gemm_rowwise's bit for bit whatever tile either takes, but the two tiles
+  // add a block's key sums in different orders, and the key mean's last bit can move a K code:
+  // 256 x 256 tiles from 512 of them on only, not where gemm_use_big also takes one round of them
+  // (1024 x 9216 x 3072 59.2 -> 38.6 us there, weights from HBM).
+  const bool big = cdiv(M, 256) * cdiv(N, 256) >= 2 * 256;
 #define MXF8_KVS_LAUNCH(Cfg, T)                                                                                    \
   launch_gemm<Cfg, MXF8_ACT_NONE, LORA_NONE, T, true>(a8, w8, sa, sw, b16, nullptr, nullptr, 0, 0.0f, o16, iM, iN, \
                                                       iK, ld_out, stream, kvs)

@@ -59,3 +59,19 @@ def test_prefixes_have_the_same_bits_on_every_tile(N, K, r, gelu):
     for m in (1, 32, 65, 130, 300, 513, 1000, 2048, 3100):
         print(f"gemm prefix {m} N={N} K={K} r={r} gelu={gelu}", flush=True)
         assert torch.equal(gemm(m), full[:m])
+
+
+@pytest.mark.parametrize("M", [1000, 1024, 1536])
+def test_kv_statistics_of_a_block_do_not_depend_on_the_rows_after_it(M):
+    """The key sums of a 128-row block are added in the order of the 128 x 128 tiles below 512
+    tiles of 256 x 256, also where the plain product takes one round of those."""
+    from minimaxh3_amd import ops
+    rng = np.random.default_rng(M)
+    C, K = 3072, 1024
+    _, _, b, (x8, sa), (w8, sw) = _operands(rng, M, 3 * C, K)
+
+    def stats(m):
+        return ops.gemm_rowwise_kv_stats(x8[:m], w8, sa[:m], sw, to_gpu(b), m, C, 2 * C, C)[1]
+
+    print(f"gemm K/V statistics M={M}", flush=True)
+    assert torch.equal(stats(M)[:, :1], stats(128))
