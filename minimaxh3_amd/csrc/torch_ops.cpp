@@ -151,6 +151,7 @@ Tensor gemm_rowwise(const Tensor& a8, const Tensor& w8, const Tensor& sa, const 
                     what, "bias must be ", N, " contiguous bf16 values");
   TORCH_CHECK_VALUE(!lora_t || (lora_b && lora_t->dim() == 2 && lora_t->size(0) == M && lora_b->dim() == 2 &&
                                 lora_b->size(0) == N && lora_b->size(1) == lora_t->size(1) &&
+                                lora_t->scalar_type() == at::kBFloat16 && lora_b->scalar_type() == at::kBFloat16 &&
                                 lora_t->is_contiguous() && lora_b->is_contiguous()),
                     what, "LoRA operands t [M, r] and B [N, r] (contiguous bf16) expected");
   const at::Device dev = a8.device();
@@ -174,7 +175,11 @@ Tensor gemm_rowwise(const Tensor& a8, const Tensor& w8, const Tensor& sa, const 
 
 Tensor lora_down(const Tensor& x_in, const Tensor& a_in) {
   require_gfx950(x_in, "lora_down");
-  TORCH_CHECK_VALUE(x_in.dim() == 2 && a_in.dim() == 2, "lora_down: expected x [M, K] and A [r, K]");
+  // (the kernel reads both as bf16 and addresses A by x's K)
+  TORCH_CHECK_VALUE(x_in.dim() == 2 && a_in.dim() == 2 && a_in.size(1) == x_in.size(1) &&
+                        x_in.scalar_type() == at::kBFloat16 && a_in.scalar_type() == at::kBFloat16,
+                    "lora_down: bf16 x [M, K] and A [r, K] expected, got ", x_in.scalar_type(), " ", x_in.sizes(),
+                    " and ", a_in.scalar_type(), " ", a_in.sizes());
   on_device(a_in, x_in.device(), "lora_down: ", "a");
   const Tensor x = x_in.stride(1) != 1 ? x_in.contiguous() : x_in, a = a_in.contiguous();
   const int64_t M = x.size(0), K = x.size(1), r = a.size(0);

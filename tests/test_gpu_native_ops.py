@@ -68,3 +68,23 @@ def test_views_vmap_and_graph_replay_equal_plain_calls():
         torch.cuda.synchronize()
         assert torch.equal(y, ref_y) and torch.equal(a, ref_a)
         assert torch.equal(mod(x), ref_y)
+
+
+@pytest.mark.parametrize("r,k,dtype", [(16, 48, torch.bfloat16), (16, 80, torch.bfloat16), (16, 64, torch.float16),
+                                       (16, 64, torch.float32), (16, 64, torch.float8_e4m3fn)])
+def test_lora_operands_of_other_widths_or_types_are_refused(r, k, dtype):
+    """The kernels read x, A, t and B as bf16 and take A's width from x: anything else is refused on the
+    host (narrower or smaller operands would be read past their end)."""
+    from minimaxh3_amd import ops
+    mod, x = _linear()
+    x8, sa = ops.quant_rows(x)
+    a = torch.zeros((r, k), device="cuda").to(dtype)
+    with pytest.raises(ValueError, match="bf16 x"):
+        ops.lora_down(x, a)
+    if dtype != torch.bfloat16:
+        with pytest.raises(ValueError, match="bf16 x"):
+            ops.lora_down(x.to(dtype), torch.zeros((r, 64), device="cuda", dtype=torch.bfloat16))
+        t, b = (torch.zeros((n, r), device="cuda", dtype=torch.bfloat16) for n in (5, 32))
+        for tt, bb in ((t.to(dtype), b), (t, b.to(dtype))):
+            with pytest.raises(ValueError, match="LoRA operands"):
+                ops.gemm_rowwise(x8, mod.w8, sa, mod.w_scale, None, 0, tt, bb, 1.0)
