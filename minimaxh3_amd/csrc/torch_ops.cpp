@@ -87,6 +87,7 @@ constexpr auto kE4M3 = at::kFloat8_e4m3fn;
 
 std::tuple<Tensor, Tensor> quant_rows(const Tensor& x_in) {
   require_gfx950(x_in, "quant_rows");
+  TORCH_CHECK_INDEX(x_in.dim() >= 2, "quant_rows: expected x [M, K], got ", x_in.dim(), " dimensions");
   TORCH_CHECK_VALUE(x_in.dim() == 2, "quant_rows: expected x [M, K]");
   const Tensor x = x_in.stride(1) != 1 || x_in.stride(0) < x_in.size(1) ? x_in.contiguous() : x_in;
   const int64_t M = x.size(0), K = x.size(1);
@@ -175,6 +176,7 @@ Tensor gemm_rowwise(const Tensor& a8, const Tensor& w8, const Tensor& sa, const 
 
 Tensor lora_down(const Tensor& x_in, const Tensor& a_in) {
   require_gfx950(x_in, "lora_down");
+  TORCH_CHECK_INDEX(x_in.dim() >= 2, "lora_down: expected x [M, K], got ", x_in.dim(), " dimensions");
   // (the kernel reads both as bf16 and addresses A by x's K)
   TORCH_CHECK_VALUE(x_in.dim() == 2 && a_in.dim() == 2 && a_in.size(1) == x_in.size(1) &&
                         x_in.scalar_type() == at::kBFloat16 && a_in.scalar_type() == at::kBFloat16,

@@ -88,3 +88,14 @@ def test_lora_operands_of_other_widths_or_types_are_refused(r, k, dtype):
         for tt, bb in ((t.to(dtype), b), (t, b.to(dtype))):
             with pytest.raises(ValueError, match="LoRA operands"):
                 ops.gemm_rowwise(x8, mod.w8, sa, mod.w_scale, None, 0, tt, bb, 1.0)
+
+
+def test_missing_dimensions_raise_index_errors():
+    """As indexing the missing dimension of x does; too many dimensions stay ValueErrors."""
+    from minimaxh3_amd import ops
+    _, x = _linear()
+    a = torch.zeros((16, 64), device="cuda", dtype=torch.bfloat16)
+    for call in (ops.quant_rows, lambda t: ops.lora_down(t, a)):
+        for bad, err in ((x[0], IndexError), (x[0, 0], IndexError), (x[None], ValueError)):
+            with pytest.raises(err):
+                call(bad)
