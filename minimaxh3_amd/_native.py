@@ -1,7 +1,7 @@
 """ctypes binding of the C ABI in include/mxf8.h (libmxf8.so, built for gfx950).
 
-The library is loaded lazily on first use.  There is no fallback: if it is missing or
-the device is not an MI355X-class gfx950 GPU, every entry point raises.
+The library is loaded on first use, or when ``ops`` is imported and it is there.  There is no
+fallback: if it is missing or the device is not an MI355X-class gfx950 GPU, every entry point raises.
 """
 from __future__ import annotations
 
@@ -65,6 +65,10 @@ class NativeError(RuntimeError):
 
 def lib_path() -> str:
     return _LIB_PATH
+
+
+def ops_path() -> str:
+    return _OPS_PATH
 
 
 def _bind(path: str):

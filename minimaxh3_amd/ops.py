@@ -6,12 +6,16 @@ torch.compile: the DiT blocks are compiled with ``fullgraph=False``
 breaks.  Outputs come from torch's caching allocator; launches go to the current stream.
 
 The ops of the hot path (quant_rows, adaln_quant_rows, gemm_rowwise, lora_down,
-attn_quant_kv, attn_fwd_q) run as native dispatcher kernels (csrc/torch_ops.cpp): their
-Python bodies only load those on the first GPU call.  The others call the C ABI from here.
+attn_quant_kv, attn_fwd_q) run as native dispatcher kernels (csrc/torch_ops.cpp), which are
+registered when this module is imported: the dispatcher reads an operator's kernels without
+a lock, so none may be added while another thread calls it.  Their Python bodies see only
+what has no native kernel: other devices, and a library built after the import.  The other
+ops call the C ABI from here.
 """
 from __future__ import annotations
 
 import math
+import os
 
 import torch
 
@@ -32,8 +36,8 @@ def _prep(t: torch.Tensor, what: str) -> None:
 
 def _native(t: torch.Tensor, what: str):
     """The native op ``mxf8::what``.  Runs when the dispatcher has no native kernel for the
-    call yet: refuses other devices, then registers the kernels, which take every later GPU
-    call before it reaches Python."""
+    call: refuses other devices, then (the library was not there at the import) registers the
+    kernels, which take every later GPU call before it reaches Python."""
     _prep(t, what)
     N.load_ops()
     return getattr(torch.ops.mxf8, what).default
@@ -412,3 +416,16 @@ def _(q, c, k8, v8t, sk, sv, key_mask, key_bias, repair_tau, Sk, kv_mode=0):
 def softmax_c(scale: float | None, D: int) -> float:
     """c = (scale or 1/sqrt(D)) * log2(e) (kernels/fp8_attention.py:315)."""
     return (scale if scale is not None else 1.0 / math.sqrt(D)) * 1.4426950408889634
+
+
+def _register() -> None:
+    """Register the native kernels, unless the library is yet to be built (or, stale, does not
+    load): then the first GPU call does, or raises."""
+    if os.path.exists(N.lib_path()) and os.path.exists(N.ops_path()):
+        try:
+            N.load_ops()
+        except (OSError, AttributeError):
+            pass
+
+
+_register()
