@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_tiles.h"
 
 namespace mxf8 {
 
@@ -88,24 +89,6 @@ __device__ __forceinline__ void bf16r2(float& a, float& b) {
 // quantizer loads on top were each slower in the chained block.
 __device__ __forceinline__ void store_out16(uint16_t* p, const uint4& v) {
   __builtin_nontemporal_store(v4i{(int)v.x, (int)v.y, (int)v.z, (int)v.w}, reinterpret_cast<v4i*>(p));
-}
-
-// Map a tile sequence number s to an output tile.  Workgroups are dealt to the 8 XCDs
-// round-robin and a persistent workgroup b walks s = b, b + G, b + 2G, ... (G = grid, a
-// multiple of 8), so s % 8 names the XCD: give every XCD a contiguous range of tile ids,
-// then walk that range in groups of group_m token-tiles so concurrently running tiles
-// share operand panels in the XCD's L2.
-__device__ __forceinline__ void tile_coords(int s, int tiles_m, int tiles_n, int group_m, int& tm, int& tn) {
-  const int nwg = tiles_m * tiles_n;
-  const int q = nwg >> 3, rem = nwg & 7, x = s & 7, j = s >> 3;
-  const int id = (x < rem ? x * (q + 1) : rem * (q + 1) + (x - rem) * q) + j;
-  const int per_group = group_m * tiles_n;
-  const int g = id / per_group;
-  const int first_m = g * group_m;
-  const int gsize = min(tiles_m - first_m, group_m);
-  const int in = id - g * per_group;
-  tm = first_m + in % gsize;
-  tn = in / gsize;
 }
 
 // Workgroup barrier that waits for this wave's LDS traffic but, unlike __syncthreads(),

@@ -58,7 +58,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_ring_kernel(
     const uint8_t* __restrict__ a8, const uint8_t* __restrict__ w8, const float* __restrict__ sa,
     const float* __restrict__ sw, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ lora_t,
     const uint16_t* __restrict__ lora_b, int lora_r, float lora_scale, uint16_t* __restrict__ out, int M, int N,
-    int K, int64_t ld_out, int tiles_m, int tiles_n) {
+    int K, int64_t ld_out, int tiles_m, int tiles_n, int group_m) {
   constexpr int TM = C::TM, TN = C::TN, NS = C::NS;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[NS * C::STAGE];
   __shared__ __attribute__((aligned(16))) float ep[C::EP];  // channel scales [BN], bias [BN], token scales [BM]
@@ -67,8 +67,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_ring_kernel(
   const int wrow0 = wn * (C::BN / C::WN), xrow0 = wm * (C::BM / C::WM);
   const int nk = (K + C::BK - 1) / C::BK;
   int tm, tn;
-  // token-tiles fastest: the workgroups that share a weight panel run on one XCD
-  tile_coords(blockIdx.x, tiles_m, tiles_n, tiles_m, tm, tn);
+  tile_coords(blockIdx.x, tiles_m, tiles_n, group_m, tm, tn);
   const int m0 = tm * C::BM, n0 = tn * C::BN;
   uint32_t lane_off[2];
 #pragma unroll
@@ -293,7 +292,7 @@ static void launch_gemm_ring(int act, const uint8_t* a8, const uint8_t* w8, cons
 #define MXF8_RING_CASE(A, L, T)                                                                                     \
   if (act == A && lora == L && ktail == T) {                                                                        \
     gemm_ring_kernel<C, A, L, T><<<dim3(tiles_m * tiles_n), dim3(C::THREADS), 0, st>>>(                             \
-        a8, w8, sa, sw, bias, lt, lb, r, ls, out, M, N, K, ld_out, tiles_m, tiles_n);                               \
+        a8, w8, sa, sw, bias, lt, lb, r, ls, out, M, N, K, ld_out, tiles_m, tiles_n, RING_GROUP_M);                 \
     return;                                                                                                         \
   }
 #define MXF8_RING_CASES(A, L) MXF8_RING_CASE(A, L, false) MXF8_RING_CASE(A, L, true)
