@@ -27,11 +27,14 @@
 #include <type_traits>
 
 #include "common.h"
+
+namespace mxf8 {
+constexpr int GEMM_BK = 128;
+}
+
 #include "gemm_tiles.h"
 
 namespace mxf8 {
-
-constexpr int GEMM_BK = 128;
 
 template <int BM_, int BN_, int WM_, int WN_>
 struct GemmCfg {
@@ -1021,7 +1024,7 @@ extern "C" int mxf8_gemm_rowwise_kv_stats(const uint8_t* a8, const uint8_t* w8, 
   const bool ktail = (K % GEMM_BK) != 0;
   // The output is mxf8_gemm_rowwise's bit for bit whatever tile either takes, but the two tiles
   // add a block's key sums in different orders, and the key mean's last bit can move a K code:
-  // 256 x 256 tiles from 512 of them on only, not where gemm_use_big also takes one round of them
+  // 256 x 256 tiles from 512 of them on only, not where gemm_pick also takes one round of them
   // (1024 x 9216 x 3072 59.2 -> 38.6 us there, weights from HBM).
   const bool big = cdiv(M, 256) * cdiv(N, 256) >= 2 * 256;
 #define MXF8_KVS_LAUNCH(Cfg, T)                                                                                    \

@@ -8,7 +8,7 @@
 // stage waits out one copy's latency (1.07 us per 128 bytes of K on MI355X, weights from
 // HBM).  Here the tile is small enough to give every CU one, the ring keeps NS - 1 stages of
 // copies in flight, and a stage's fragments are read from LDS while the previous stage's
-// products run, so a stage costs 0.25-0.7 us (by tile size, gemm_pick).  MI355X, weights
+// products run, so a stage costs 0.25-0.55 us (by tile size, gemm_pick).  MI355X, weights
 // from HBM, before -> after: 1 x 3072 x 3072 16.7 -> 8.0 us, 512 x 3072 x 3072 18.9 -> 11.7,
 // 1 x 9216 x 3072 23.2 -> 10.3, 256 x 9216 x 3072 26.6 -> 19.9, 1 x 3072 x 12288 83.6 -> 23.6,
 // 1024 x 3072 x 12288 103.7 -> 64.7 us.  Splitting K over workgroups would shorten the chain
@@ -214,74 +214,12 @@ __global__ __launch_bounds__(C::THREADS) void gemm_ring_kernel(
   }
 }
 
-// ---- dispatch -------------------------------------------------------------------------
+// ---- dispatch (gemm_pick chooses) ------------------------------------------------------
 // Tiles of the ring kernel, smallest first.
 typedef GemmRing<32, 64, 1, 2, 4, 2> GemmRing32x64;     // 96 KB of LDS: one workgroup per CU
 typedef GemmRing<64, 64, 2, 2, 4, 1> GemmRing64x64;     // 64 KB: two
 typedef GemmRing<128, 64, 4, 2, 3, 1> GemmRing128x64;   // 72 KB: two
 typedef GemmRing<128, 128, 2, 4, 4, 1> GemmRing128x128; // 128 KB: one
-
-// Estimated time (us) of `tiles` workgroups, `per_cu` of them resident on a CU, over ns
-// 128-byte stages of K: a start-up cost, then per round t1 per stage with one workgroup on a
-// CU or t2 with two, and the LoRA branch's `lora` per workgroup on a CU.
-inline float gemm_time(int64_t tiles, int cus, int per_cu, int64_t ns, float start, float t1, float t2, float lora) {
-  if (per_cu == 1) return start + (float)cdiv(tiles, cus) * (t1 * (float)ns + lora);
-  const int64_t full = tiles / (2 * cus), rem = tiles - full * 2 * cus;
-  return start + (float)full * (t2 * (float)ns + 2.0f * lora) +
-         (rem == 0 ? 0.0f : rem <= cus ? t1 * (float)ns + lora : t2 * (float)ns + 2.0f * lora);
-}
-
-// The 128 x 128 tiles of gemm_fp8_rowwise_kernel (two stage buffers; long-K panels share the
-// L2s less).  r: LoRA rank, 0 without; the LoRA costs them 1 us per 64 ranks from LDS
-// (r <= 128) or 2.4 from global memory.
-inline float gemm_time_small(int64_t M, int64_t N, int64_t K, int64_t r, int cus) {
-  return gemm_time(cdiv(M, 128) * cdiv(N, 128), cus, 2, cdiv(K, GEMM_BK), 2.25f, K < 8192 ? 0.78f : 1.0f,
-                   K < 8192 ? 1.16f : 1.12f, (r <= 128 ? 1.0f : 2.4f) * (float)r / 64.0f);
-}
-
-// Whether the 256 x 256 tiles take an M x N x K product whose best other tile is estimated at
-// `other` us: always from 512 of them on; and where they make one round over the CUs and save a
-// tenth or more of the estimate, 1.4 us per stage against the part-filled second round of the
-// smaller ones.  MI355X, weights from HBM / from the MALL, 128 x 128 -> 256 x 256 tiles:
-// 1024 x 9216 x 3072 59.2 -> 38.6 / 40.4 -> 33.4 us, 1536 x 9216 x 3072 59.4 -> 41.6 / 44.9 -> 38.2,
-// 2048 x 6144 x 3072 56.1 -> 39.9 / 41.6 -> 35.7, 3072 x 3072 x 3072 44.7 -> 37.5 / 40.8 -> 33.7,
-// 3072 x 3072 x 12288 179.8 -> 145.7 / 158.4 -> 115.3.  Two rounds of them (257 to 511 tiles)
-// gained with cold weights and lost with warm ones (2048 x 9216 x 3072 87.2 -> 73.2 / 62.6 -> 71.5)
-// and keep the 128 x 128 tiles.
-inline bool gemm_use_big(int64_t M, int64_t N, int64_t K, int64_t r, int cus, float other) {
-  const int64_t tiles = cdiv(M, 256) * cdiv(N, 256);
-  if (tiles >= 2 * 256) return true;
-  return tiles <= cus &&
-         gemm_time(tiles, cus, 1, cdiv(K, GEMM_BK), 3.0f, 1.4f, 0.0f, 2.0f * (float)r / 64.0f) <= 0.9f * other;
-}
-
-// The tile of an M x N x K product: 0-3 a ring tile in the order above, else 128 x 128 or
-// 256 x 256 tiles of gemm_fp8_rowwise_kernel.  The constants of the ring tiles and the
-// 128 x 128 ones are fitted to MI355X times of 210 products (M 1-6144; N x K from 64 x 2048 to
-// 18432 x 3072 and 3072 x 12288; weights from HBM; graph replays).  Over those the ring tiles and
-// the 128 x 128 ones together took 1.48 times less than the 128 x 128 ones alone in geometric
-// mean, 2% longer than the best tile each time; the large gains are where M <= 1280 leaves CUs
-// without a 128 x 128 tile.  Past that the larger tile reads fewer operand bytes from the L2s
-// and wins (2048 x 3072 x 3072: 22.6 us against 29.2 with 128 x 64).  A LoRA costs the ring
-// tiles 0.5-3.7 us per 64 ranks, read from global memory in the epilogue (1024 x 3072 x 3072,
-// rank 128: 22.4 us with 128 x 128 tiles of the other kernel against 24.0).
-enum { GEMM_TILE_128 = 4, GEMM_TILE_256 = 5 };
-inline int gemm_pick(int64_t M, int64_t N, int64_t K, int64_t r, int cus) {
-  const int64_t ns = cdiv(K, GEMM_BK);
-  const float l = (float)r / 64.0f;
-  auto tiles = [&](int bm, int bn) { return cdiv(M, bm) * cdiv(N, bn); };
-  const float small = gemm_time_small(M, N, K, r, cus);
-  const float t[4] = {gemm_time(tiles(32, 64), cus, 1, ns, 2.5f, 0.29f, 0.0f, 0.5f * l),
-                      gemm_time(tiles(64, 64), cus, 2, ns, 3.0f, 0.315f, 0.55f, 1.1f * l),
-                      gemm_time(tiles(128, 64), cus, 2, ns, 2.3f, 0.415f, 0.83f, 2.0f * l),
-                      gemm_time(tiles(128, 128), cus, 1, ns, 2.1f, 0.66f, 0.0f, 3.7f * l)};
-  int best = 0;
-  for (int i = 1; i < 4; ++i)
-    if (t[i] < t[best]) best = i;
-  const bool ring = t[best] <= 0.95f * small;
-  if (gemm_use_big(M, N, K, r, cus, ring ? t[best] : small)) return GEMM_TILE_256;
-  return ring ? best : GEMM_TILE_128;
-}
 
 template <class C>
 static void launch_gemm_ring(int act, const uint8_t* a8, const uint8_t* w8, const float* sa,
