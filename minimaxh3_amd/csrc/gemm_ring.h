@@ -33,7 +33,7 @@ struct GemmRing {
   static_assert(NS * STAGE + EP * 4 <= 160 * 1024, "LDS ring");
   static_assert(BM * OUT_PITCH <= NS * STAGE, "output staging");
   static_assert((BM + BN) / 8 % NW == 0 && BN % 16 == 0, "DMA shares");
-  static_assert(NS >= 3 && (NS - 2) * DMA_PER_WAVE < 64, "ring depth");
+  static_assert(NS >= 3 && (NS - 1) * DMA_PER_WAVE < 64, "vmcnt counts the copies of NS - 1 stages");
 
   // This wave's share of one stage, as gemm_dma, but whichever operand each instruction's 8
   // rows belong to.

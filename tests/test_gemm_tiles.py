@@ -117,3 +117,14 @@ def test_pick_is_near_the_best_measured_tile(pick, shape):
                                    (77648, 3072, 3072, 4096), (8192, 4096, 512, 0)])
 def test_512_tiles_of_256_always_take_them(pick, shape):
     assert pick(*shape) == 5
+
+
+@pytest.mark.parametrize("ring,fits", [("32, 64, 1, 2, 4, 2", True), ("32, 64, 1, 1, 4, 2", False)])
+def test_ring_depth_is_bounded_by_the_copy_counter(ring, fits):
+    """The first stage is waited for with NS - 1 later stages' copies in flight, and the counter
+    holds 63: 36 of them, and 72 with one wave, which must not compile."""
+    code = f'#include "gemm.hip"\nstatic_assert(mxf8::GemmRing<{ring}>::NS == 4, "");\n'
+    res = subprocess.run([build.hipcc(), "--offload-arch=gfx950", "--offload-host-only", "-std=c++17", "-fsyntax-only",
+                          "-I", build.CSRC, "-x", "hip", "-"], input=code, capture_output=True, text=True)
+    assert (res.returncode == 0) == fits, res.stderr[-2000:]
+    assert fits or "counts the copies" in res.stderr
