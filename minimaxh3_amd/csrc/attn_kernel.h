@@ -474,6 +474,15 @@ constexpr bool attn_scores_scaled() {
 constexpr int kScoreScaleE8M0 = 127 - 96;
 constexpr float kScoreScale = 0x1p-96f;
 
+// Single-precision denormals of this wave's VALU (MODE bits 5:4): bit 0 lets denormal inputs
+// through, bit 1 denormal results.  (Volatile asm, which stays in order with the asm
+// statements between two calls; the builtin's instruction may move across them.  Other
+// instructions are kept off by scheduling barriers around the pair.)
+template <int BITS>
+__device__ __forceinline__ void set_f32_denorm() {
+  asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 4, 2), %0" ::"n"(BITS));
+}
+
 // The exp2-free P codes of one tile without the repair: word 4 (t & 1) + w4 of the PV B
 // operand of key half t >> 1 holds scores 4 w4 .. 4 w4 + 3 of subtile t.
 //
@@ -496,69 +505,58 @@ constexpr float kScoreScale = 0x1p-96f;
 // bit for bit over 10^8 scores, boundaries of the flush among them (where exact bits below 8
 // round to 8 the code is now 8, as the reference's test of the rounded value gives).
 //
-// Nothing but the FMAs may run while denormal results are flushed (MODE bits 5:4 hold the
-// denormal mode of fp32: bit 0 lets denormal inputs through, bit 1 denormal results), and what
-// reads a byte write needs wait states that the compiler does not know of.  So one asm
-// statement, in which the compiler can place nothing, makes the codes of one key half from
-// the mode change to the wait states: a word's next byte is written four instructions after
-// the last (one wait state is needed), and the s_nop at the end covers the last writes before
-// any reader, a matrix product (two wait states) included.  Every score was read by
+// Nothing but the FMAs may run while denormal results are flushed: volatile asm keeps them
+// between the two mode changes, and scheduling barriers keep every other instruction outside
+// (without them integer instructions did move in).  What reads a byte write needs wait states
+// that the compiler does not know of: a word's next byte is written four instructions after
+// the last (one wait state is needed), and each multiply statement ends with an s_nop that
+// covers its last writes before any reader, a matrix product (two wait states) included.
+// tests/test_attn_codes_asm.py reads both off the compiled kernels.  Every score was read by
 // attn_part_max before, so none is still being written by a matrix product.
 //
-// y goes to registers of its own: written over the scores it cost 1-2% at 480p, in copies
-// around the statement, and so did 64 scores in one statement; this form and one statement
-// per instruction measured the same (20280 tokens 2223 and 2218 us, two joint items 5168).
+// The FMAs stay one statement each, which leaves the compiler their registers: 32 with their
+// multiplies in one statement needs y beside the scores, and at D = 64 a third wave per SIMD no
+// longer fits (24 heads of 16000 tokens with a mask 1427 -> 1674 us); with 16 per statement it
+// took 1456 us, with 64 in place 1451.
 template <bool HAS_BIAS>
 __device__ __forceinline__ void attn_codes_tile(const v16f (&s)[4], float sq, float skj, float csty, v8i (&p)[2]) {
-  const float cy = HAS_BIAS ? 0x1p-126f : (sq * skj) * (0x1p-126f / kScoreScale);
-  const float cr = 0x1p-20f;
-// operands: %0-%7 the words, %8-%39 y, %40-%71 the scores, %72 cy, %73 csty, %74 2^-20
-#define MXF8_SET_F32_DENORM(BITS) "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 4, 2), " #BITS "\n"
-#define MXF8_FMA(Y, S) "v_fma_f32 %" #Y ", %" #S ", %72, %73 clamp\n"
-#define MXF8_MUL(W, Y) "v_mul_f32 %" #W ", %74, %" #Y "\n"
+  float cy = HAS_BIAS ? 0x1p-126f : (sq * skj) * (0x1p-126f / kScoreScale);
+  float cr = 0x1p-20f;
+  float y[4][16];
+  asm volatile("" : "+v"(cy), "+v"(csty), "+v"(cr));
+  __builtin_amdgcn_sched_barrier(0);
+  set_f32_denorm<1>();
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      asm volatile("v_fma_f32 %0, %1, %2, %3 clamp" : "=v"(y[t][i]) : "v"(s[t][i]), "v"(cy), "v"(csty));
+  set_f32_denorm<3>();
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    uint32_t w[4];
+    const float(&u)[16] = y[t];
 #define MXF8_MUL_BYTE(B, W, Y) \
-  "v_mul_f32_sdwa %" #W ", %74, %" #Y " dst_sel:BYTE_" #B " dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD\n"
-#define MXF8_X8(C, X, I) \
-  C(X[I]), C(X[I + 1]), C(X[I + 2]), C(X[I + 3]), C(X[I + 4]), C(X[I + 5]), C(X[I + 6]), C(X[I + 7])
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const v16f &s0 = s[2 * h], &s1 = s[2 * h + 1];
-    uint32_t w[8];
-    float y[32];
+  "v_mul_f32_sdwa %" #W ", %4, %" #Y " dst_sel:BYTE_" #B " dst_unused:UNUSED_PRESERVE src0_sel:DWORD src1_sel:DWORD\n"
     asm volatile(
+        "v_mul_f32 %0, %4, %5\n"
+        "v_mul_f32 %1, %4, %9\n"
+        "v_mul_f32 %2, %4, %13\n"
+        "v_mul_f32 %3, %4, %17\n"
         // clang-format off
-        MXF8_SET_F32_DENORM(1)
-        MXF8_FMA(8, 40) MXF8_FMA(9, 41) MXF8_FMA(10, 42) MXF8_FMA(11, 43)
-        MXF8_FMA(12, 44) MXF8_FMA(13, 45) MXF8_FMA(14, 46) MXF8_FMA(15, 47)
-        MXF8_FMA(16, 48) MXF8_FMA(17, 49) MXF8_FMA(18, 50) MXF8_FMA(19, 51)
-        MXF8_FMA(20, 52) MXF8_FMA(21, 53) MXF8_FMA(22, 54) MXF8_FMA(23, 55)
-        MXF8_FMA(24, 56) MXF8_FMA(25, 57) MXF8_FMA(26, 58) MXF8_FMA(27, 59)
-        MXF8_FMA(28, 60) MXF8_FMA(29, 61) MXF8_FMA(30, 62) MXF8_FMA(31, 63)
-        MXF8_FMA(32, 64) MXF8_FMA(33, 65) MXF8_FMA(34, 66) MXF8_FMA(35, 67)
-        MXF8_FMA(36, 68) MXF8_FMA(37, 69) MXF8_FMA(38, 70) MXF8_FMA(39, 71)
-        MXF8_SET_F32_DENORM(3)
-        MXF8_MUL(0, 8) MXF8_MUL(1, 12) MXF8_MUL(2, 16) MXF8_MUL(3, 20)
-        MXF8_MUL_BYTE(1, 0, 9) MXF8_MUL_BYTE(1, 1, 13) MXF8_MUL_BYTE(1, 2, 17) MXF8_MUL_BYTE(1, 3, 21)
-        MXF8_MUL_BYTE(2, 0, 10) MXF8_MUL_BYTE(2, 1, 14) MXF8_MUL_BYTE(2, 2, 18) MXF8_MUL_BYTE(2, 3, 22)
-        MXF8_MUL_BYTE(3, 0, 11) MXF8_MUL_BYTE(3, 1, 15) MXF8_MUL_BYTE(3, 2, 19) MXF8_MUL_BYTE(3, 3, 23)
-        MXF8_MUL(4, 24) MXF8_MUL(5, 28) MXF8_MUL(6, 32) MXF8_MUL(7, 36)
-        MXF8_MUL_BYTE(1, 4, 25) MXF8_MUL_BYTE(1, 5, 29) MXF8_MUL_BYTE(1, 6, 33) MXF8_MUL_BYTE(1, 7, 37)
-        MXF8_MUL_BYTE(2, 4, 26) MXF8_MUL_BYTE(2, 5, 30) MXF8_MUL_BYTE(2, 6, 34) MXF8_MUL_BYTE(2, 7, 38)
-        MXF8_MUL_BYTE(3, 4, 27) MXF8_MUL_BYTE(3, 5, 31) MXF8_MUL_BYTE(3, 6, 35) MXF8_MUL_BYTE(3, 7, 39)
-        "s_nop 1\n"
+        MXF8_MUL_BYTE(1, 0, 6) MXF8_MUL_BYTE(1, 1, 10) MXF8_MUL_BYTE(1, 2, 14) MXF8_MUL_BYTE(1, 3, 18)
+        MXF8_MUL_BYTE(2, 0, 7) MXF8_MUL_BYTE(2, 1, 11) MXF8_MUL_BYTE(2, 2, 15) MXF8_MUL_BYTE(2, 3, 19)
+        MXF8_MUL_BYTE(3, 0, 8) MXF8_MUL_BYTE(3, 1, 12) MXF8_MUL_BYTE(3, 2, 16) MXF8_MUL_BYTE(3, 3, 20)
         // clang-format on
-        : MXF8_X8("=&v", w, 0), MXF8_X8("=&v", y, 0), MXF8_X8("=&v", y, 8), MXF8_X8("=&v", y, 16),
-          MXF8_X8("=&v", y, 24)
-        : MXF8_X8("v", s0, 0), MXF8_X8("v", s0, 8), MXF8_X8("v", s1, 0), MXF8_X8("v", s1, 8), "v"(cy), "v"(csty),
-          "s"(cr));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) p[h][i] = (int)w[i];
-  }
-#undef MXF8_X8
+        "s_nop 1\n"
+        : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3])
+        : "v"(cr), "v"(u[0]), "v"(u[1]), "v"(u[2]), "v"(u[3]), "v"(u[4]), "v"(u[5]), "v"(u[6]), "v"(u[7]), "v"(u[8]),
+          "v"(u[9]), "v"(u[10]), "v"(u[11]), "v"(u[12]), "v"(u[13]), "v"(u[14]), "v"(u[15]));
 #undef MXF8_MUL_BYTE
-#undef MXF8_MUL
-#undef MXF8_FMA
-#undef MXF8_SET_F32_DENORM
+#pragma unroll
+    for (int w4 = 0; w4 < 4; ++w4) p[t >> 1][4 * (t & 1) + w4] = (int)w[w4];
+  }
 }
 
 // Per-tile constants of the code arithmetic with the repair (see attn_codes_w4).
