@@ -642,8 +642,8 @@ __global__ __launch_bounds__(256) void attn_quant_v_kernel(const void* __restric
 // ---------------------------------------------------------------------------------------
 // K and V of one attention together (kernels/fp8_attention.py:338-369): one pass over both
 // for the statistics that need the whole sequence (the key mean, the per-channel V amax),
-// one fold of both (for few keys inside the quantizing blocks, kv_fold_in_quant), then one
-// launch that quantizes a 128-key tile of K or of V per block.
+// one fold of both (for few keys inside the quantizing blocks, kv_split), then one launch that
+// quantizes a 128-key tile of K and of V per block (for few keys of one of them).
 // The second read of K and V follows the first closely, so it is mostly served by the
 // MALL; in the fused QKV layout ([B, S, 2, H, D]) the two reads of a key's K and V rows
 // are adjacent.
@@ -736,39 +736,31 @@ __global__ __launch_bounds__(256) void attn_kv_fold_kernel(const float* __restri
   }
 }
 
-// Quantizes the K tile (even blockIdx.x) or the V tile (odd) of 128 keys of one head (grid
-// (2 B*H, Skp/128)): heads fastest, so the blocks that run together read the same keys' rows,
-// and K and V in blocks of their own, which halves the chain of loads, statistics, codes and
-// stores that a launch of few tiles consists of.
+// Quantizes the K and the V tile of 128 keys of one head, heads fastest, so the blocks that run
+// together read the same keys' rows.
+//
+// SPLIT: K (even blockIdx.x) and V (odd) in blocks of their own (grid (2 B*H, Skp/128)), which
+// halves the chain of loads, statistics, codes and stores that a launch of few tiles consists
+// of; otherwise (grid (B*H, Skp/128)) a block does one after the other (see kv_split).
 //
 // FOLD: the block folds its head's statistic from the partial slabs itself (every block of a
 // head the same way, attn_kv_fold_kernel's order and so its bits), and the head's first block
 // writes it out: no fold launch.
-template <int DT, int D, bool VECK, bool VECV, bool FOLD>
+template <int DT, int D, bool VECK, bool VECV, bool SPLIT, bool FOLD>
 __global__ __launch_bounds__(256) void attn_quant_kv_kernel(const void* __restrict__ k, Strides4 stk,
                                                             const void* __restrict__ v, Strides4 stv, int64_t H,
                                                             int64_t S, int64_t Sp, const float* __restrict__ part,
                                                             int nch, float* __restrict__ mean, float* __restrict__ sv,
                                                             uint8_t* __restrict__ k8, float* __restrict__ sk,
                                                             uint8_t* __restrict__ v8t) {
+  static_assert(SPLIT || !FOLD, "the fold is for launches of few tiles");
   __shared__ float red[FOLD ? 256 : 4];
   __shared__ float stat[FOLD ? D : 1];
   __shared__ QuantVLds<D> L;
-  const int64_t bh = blockIdx.x >> 1, blk = blockIdx.y, nb = gridDim.y, BH = gridDim.x >> 1;
-  if (blockIdx.x & 1) {
-    quant_v_tile<DT, D, VECV>(v, stv, H, S, Sp, [&]() -> const float* {
-      if constexpr (FOLD) {
-        const float amax = colfold<D, true>(part + BH * nch * D, nch, bh, red);
-        if (threadIdx.x < D) {
-          stat[threadIdx.x] = e4m3_scale(amax);
-          if (blk == 0) sv[bh * D + threadIdx.x] = stat[threadIdx.x];
-        }
-        return stat;  // (a thread reads only what it wrote)
-      } else {
-        return sv + bh * D;
-      }
-    }, v8t, blk, bh, L);
-  } else {
+  const int64_t bh = SPLIT ? blockIdx.x >> 1 : blockIdx.x, BH = SPLIT ? gridDim.x >> 1 : gridDim.x;
+  const int64_t blk = blockIdx.y, nb = gridDim.y;
+  const bool is_v = SPLIT && (blockIdx.x & 1);
+  if (!is_v)
     quant_qk_tile<DT, D, true, VECK>(k, stk, H, S, Sp, 0.0f, [&]() -> const float* {
       if constexpr (FOLD) {
         const float sum = colfold<D, false>(part, nch, bh, red);
@@ -782,7 +774,19 @@ __global__ __launch_bounds__(256) void attn_quant_kv_kernel(const void* __restri
         return mean + bh * D;
       }
     }, k8, sk, blk, bh, nb, red);
-  }
+  if (!SPLIT || is_v)
+    quant_v_tile<DT, D, VECV>(v, stv, H, S, Sp, [&]() -> const float* {
+      if constexpr (FOLD) {
+        const float amax = colfold<D, true>(part + BH * nch * D, nch, bh, red);
+        if (threadIdx.x < D) {
+          stat[threadIdx.x] = e4m3_scale(amax);
+          if (blk == 0) sv[bh * D + threadIdx.x] = stat[threadIdx.x];
+        }
+        return stat;  // (a thread reads only what it wrote)
+      } else {
+        return sv + bh * D;
+      }
+    }, v8t, blk, bh, L);
 }
 
 // Fold of the K/V column statistics that the QKV projection's epilogue emits
@@ -1070,13 +1074,14 @@ extern "C" int64_t mxf8_attn_kv_workspace_bytes(int64_t B, int64_t H, int64_t S,
   return (2 * (int64_t)colreduce_chunks(BH, S) + 1) * BH * D * (int64_t)sizeof(float);
 }
 
-// Whether the quantizing blocks fold the statistics themselves: every one of the B*H*nb pairs
-// reads its head's slabs again (2 nch D floats from the L2), against one fold launch.  MI355X,
-// 24 heads, D = 128, all launches, folded there / in a launch of their own: 1024 keys (3 MB of
-// re-reads) 12.5 / 14.8 us, 4673 keys (58 MB) 31.3 / 33.5, 20280 keys (250 MB) 115.5 / 107.7.
-static bool kv_fold_in_quant(int64_t BH, int64_t nb, int nch, int64_t D) {
-  return BH * nb * nch * 2 * D * (int64_t)sizeof(float) <= ((int64_t)64 << 20);
-}
+// Whether K and V take blocks of their own, which fold the statistics themselves: where all of
+// them are resident together (8 per CU).  Past that the last, part-filled round of blocks costs
+// more than the shorter chain saves, and every block would read its head's slabs again
+// (2 nch D floats from the L2), against one fold launch.  MI355X, D = 128, all launches, split and
+// folded / neither: 24 x 1024 keys (384 blocks) 12.7 / 15.1 us, 24 x 4096 (1536) 29.5 / 30.5,
+// 24 x 5000 (1920) 34.8 / 34.4; 40 x 4096 (2560) 46.5 / 43.5, 96 x 3000 (4608) 82.1 / 76.6,
+// 24 x 20280 (7632) 115.5 / 107.7; split alone 24 x 6000 (2256) 43.2 / 40.8.
+static bool kv_split(int64_t BH, int64_t nb) { return 2 * BH * nb <= 8 * (int64_t)device_cus(); }
 
 template <int DT, int D>
 static void launch_kv(const void* k, const Strides4& stk, bool veck, const void* v, const Strides4& stv, bool vecv,
@@ -1085,19 +1090,17 @@ static void launch_kv(const void* k, const Strides4& stk, bool veck, const void*
   const int64_t rpc = cdiv(S, nch);
   const dim3 rgrid((unsigned)BH, (unsigned)nch);
   const int64_t nb = cdiv(S, 128);
-  const dim3 qgrid((unsigned)(2 * BH), (unsigned)nb);
-  const bool fold = kv_fold_in_quant(BH, nb, nch, D);
 #define MXF8_KV_CASE(VK, VV)                                                                                     \
   if (veck == VK && vecv == VV) {                                                                                \
     attn_kv_colreduce_kernel<DT, D, VK, VV><<<rgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, rpc, part);         \
-    if (fold) {                                                                                                  \
-      attn_quant_kv_kernel<DT, D, VK, VV, true><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128, part, \
-                                                                            nch, mean, sv, k8, sk, v8t);         \
+    if (kv_split(BH, nb)) {                                                                                      \
+      attn_quant_kv_kernel<DT, D, VK, VV, true, true><<<dim3((unsigned)(2 * BH), (unsigned)nb), 256, 0, stream>>>( \
+          k, stk, v, stv, H, S, nb * 128, part, nch, mean, sv, k8, sk, v8t);                                     \
       return;                                                                                                    \
     }                                                                                                            \
     attn_kv_fold_kernel<D><<<dim3((unsigned)BH), 256, 0, stream>>>(part, nch, S, mean, sv);                       \
-    attn_quant_kv_kernel<DT, D, VK, VV, false><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128, nullptr, \
-                                                                           0, mean, sv, k8, sk, v8t);            \
+    attn_quant_kv_kernel<DT, D, VK, VV, false, false><<<dim3((unsigned)BH, (unsigned)nb), 256, 0, stream>>>(      \
+        k, stk, v, stv, H, S, nb * 128, nullptr, 0, mean, sv, k8, sk, v8t);                                      \
     return;                                                                                                      \
   }
   MXF8_KV_CASE(true, true)
@@ -1113,23 +1116,26 @@ static void launch_quant_kv_only(const void* k, const Strides4& stk, bool veck, 
                                  bool vecv, int64_t H, int64_t S, int64_t BH, float* mean, float* sv,
                                  uint8_t* k8, float* sk, uint8_t* v8t, hipStream_t stream) {
   const int64_t nb = cdiv(S, 128);
-  const dim3 qgrid((unsigned)(2 * BH), (unsigned)nb);
-#define MXF8_KVQ_CASE(VK, VV)                                                                                    \
-  if (veck == VK && vecv == VV) {                                                                                \
-    attn_quant_kv_kernel<DT, D, VK, VV, false><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128, nullptr, \
-                                                                           0, mean, sv, k8, sk, v8t);            \
-    return;                                                                                                      \
+  const bool split = kv_split(BH, nb);
+  const dim3 qgrid((unsigned)(split ? 2 * BH : BH), (unsigned)nb);
+#define MXF8_KVQ_CASE(VK, VV, SP)                                                                              \
+  if (veck == VK && vecv == VV && split == SP) {                                                               \
+    attn_quant_kv_kernel<DT, D, VK, VV, SP, false><<<qgrid, 256, 0, stream>>>(k, stk, v, stv, H, S, nb * 128,  \
+                                                                              nullptr, 0, mean, sv, k8, sk, v8t); \
+    return;                                                                                                    \
   }
-  MXF8_KVQ_CASE(true, true)
-  MXF8_KVQ_CASE(true, false)
-  MXF8_KVQ_CASE(false, true)
-  MXF8_KVQ_CASE(false, false)
+#define MXF8_KVQ_CASES(VK, VV) MXF8_KVQ_CASE(VK, VV, true) MXF8_KVQ_CASE(VK, VV, false)
+  MXF8_KVQ_CASES(true, true)
+  MXF8_KVQ_CASES(true, false)
+  MXF8_KVQ_CASES(false, true)
+  MXF8_KVQ_CASES(false, false)
+#undef MXF8_KVQ_CASES
 #undef MXF8_KVQ_CASE
 }
 
 // K and V quantized together: the key mean, the K quantizer, the per-channel V scale and
 // the transposed V quantizer (kernels/fp8_attention.py:338-369) in three launches, two
-// where kv_fold_in_quant puts the fold into the last.
+// where kv_split puts the fold into the last.
 static int attn_quant_kv_impl(const char* what, const void* k, const int64_t k_strides[4], const void* v,
                               const int64_t v_strides[4], int dtype, int64_t B, int64_t H, int64_t S, int64_t D,
                               uint8_t* k8, float* sk, uint8_t* v8t, float* sv, float* mean, float* part, int nch,

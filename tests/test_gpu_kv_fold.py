@@ -1,5 +1,5 @@
 """attn_quant_kv where its statistics are folded in the quantizing blocks and where a launch of
-its own folds them (kv_fold_in_quant): the separate quantizers' bits either way."""
+its own folds them (kv_split): the separate quantizers' bits either way."""
 import pytest
 import torch
 
@@ -8,9 +8,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("B,H,S,D,dtype", [
     (1, 1, 1, 128, torch.bfloat16), (2, 3, 129, 64, torch.float16), (1, 24, 1024, 128, torch.bfloat16),
-    (1, 2, 65536, 128, torch.bfloat16),   # 64 MB of slab re-reads: the last folded in the blocks
-    (1, 2, 65537, 128, torch.bfloat16),   # the first with a fold launch
-    (2, 2, 66000, 64, torch.bfloat16),
+    (1, 2, 65536, 128, torch.bfloat16),   # 2048 blocks, 8 per CU: the last with K and V split and folded
+    (1, 2, 65537, 128, torch.bfloat16),   # the first with a fold launch and one block for both
+    (2, 2, 66000, 64, torch.bfloat16), (4, 24, 1400, 128, torch.float16),   # few keys, more blocks than that
 ])
 def test_fold_in_blocks_or_launch_gives_the_same_bits(B, H, S, D, dtype):
     print(f"kv fold B={B} H={H} S={S} D={D} {dtype}", flush=True)
