@@ -99,3 +99,56 @@ def test_missing_dimensions_raise_index_errors():
         for bad, err in ((x[0], IndexError), (x[0, 0], IndexError), (x[None], ValueError)):
             with pytest.raises(err):
                 call(bad)
+
+
+def test_both_attention_ops_refuse_the_same_operands():
+    """attn_fwd checks its codes and key operands in Python, attn_fwd_q natively: the same calls are
+    refused, with the operand's name, and the same accepted."""
+    from minimaxh3_amd import ops
+    B, H, S, D, Sk = 2, 2, 130, 64, 200
+    q, k, v = (torch.randn((B, H, n, D), device="cuda", dtype=torch.bfloat16) for n in (S, Sk, Sk))
+    c = ops.softmax_c(None, D)
+    q8, sq = ops.attn_quant_q(q, c)
+    k8, sk, v8t, sv, _ = ops.attn_quant_kv(k, v)
+    mask, bias = torch.ones((B, Sk), device="cuda", dtype=torch.bool), torch.zeros((B, Sk), device="cuda")
+
+    def both(Sk=Sk, mask=None, bias=None, **codes):
+        a = {"k8": k8, "v8t": v8t, "sk": sk, "sv": sv, **codes}
+        for call in (lambda: ops.attn_fwd(q8, a["k8"], a["v8t"], sq, a["sk"], a["sv"], mask, bias, -1.0, q, Sk),
+                     lambda: ops.attn_fwd_q(q, c, a["k8"], a["v8t"], a["sk"], a["sv"], mask, bias, -1.0, Sk)):
+            yield call
+
+    for kw, name in [({"Sk": 300}, "k8"), ({"Sk": 100}, "k8"), ({"k8": k8.view(torch.uint8)}, "k8"),
+                     ({"k8": k8.transpose(2, 3)}, "k8"), ({"v8t": v8t[..., :128]}, "v8t"), ({"v8t": v8t.cpu()}, "v8t"),
+                     ({"sk": sk.double()}, "sk"), ({"sk": sk[:, :1]}, "sk"), ({"sv": sv[..., :32]}, "sv"),
+                     ({"sv": sv.half()}, "sv"), ({"mask": mask[:, :7]}, "key_mask"), ({"mask": mask.cpu()}, "key_mask"),
+                     ({"bias": bias[:, 1:]}, "key_bias"), ({"bias": bias.cpu()}, "key_bias")]:
+        for call in both(**kw):
+            with pytest.raises(ValueError, match=name):
+                call()
+    ref = None
+    for kw in ({}, {"mask": mask}, {"mask": mask[0]}, {"mask": mask.float()}, {"bias": bias}, {"bias": bias[:1]},
+               {"bias": bias.half()}, {"mask": mask.view(B, 1, 1, Sk)}):
+        outs = [call() for call in both(**kw)]
+        ref = outs[0] if ref is None else ref
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], ref)
+
+
+def test_the_fused_layout_is_the_one_the_caller_tests():
+    """ops.attn_fwd_q_supported, which the Python caller asks, and the native op agree on q's layouts."""
+    from minimaxh3_amd import ops
+    B, H, S, D = 1, 2, 40, 64
+    k = torch.randn((B, H, S, D), device="cuda", dtype=torch.bfloat16)
+    k8, sk, v8t, sv, _ = ops.attn_quant_kv(k, k)
+    qs = [k, k.half(), k.float(), k[0], k.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2),
+          torch.randn((B, S, H, D), device="cuda").bfloat16().permute(0, 2, 1, 3),
+          torch.randn((B, H, S, D + 4), device="cuda").bfloat16()[..., :D],
+          torch.randn((B, H, S, D + 8), device="cuda").bfloat16()[..., :D],
+          torch.randn((B, H, S, 2 * D), device="cuda").bfloat16()[..., ::2]]
+    for q in qs:
+        if ops.attn_fwd_q_supported(q):
+            assert ops.attn_fwd_q(q, 0.1, k8, v8t, sk, sv, None, None, -1.0, S).shape == q.shape
+        else:
+            with pytest.raises(ValueError, match="q must be"):
+                ops.attn_fwd_q(q, 0.1, k8, v8t, sk, sv, None, None, -1.0, S)
+    assert [ops.attn_fwd_q_supported(q) for q in qs] == [True, True, False, False, False, True, False, True, False]
