@@ -248,6 +248,9 @@ def attn_quant_k(k: torch.Tensor, mean: torch.Tensor) -> tuple[torch.Tensor, tor
     _prep(k, "attn_quant_k")
     B, H, S, D = k.shape
     nk = _cdiv(S, 128)
+    _on(mean, k.device, "attn_quant_k: mean")
+    if mean.numel() != B * H * D:
+        raise ValueError(f"attn_quant_k: mean must hold B*H*D = {B * H * D} values, got shape {tuple(mean.shape)}")
     mean = mean.to(torch.float32).contiguous()
     k8 = torch.empty((B, H, nk * 128, D), dtype=E4M3, device=k.device)
     sk = torch.empty((B, H, nk), dtype=torch.float32, device=k.device)

@@ -152,3 +152,16 @@ def test_the_fused_layout_is_the_one_the_caller_tests():
             with pytest.raises(ValueError, match="q must be"):
                 ops.attn_fwd_q(q, 0.1, k8, v8t, sk, sv, None, None, -1.0, S)
     assert [ops.attn_fwd_q_supported(q) for q in qs] == [True, True, False, False, False, True, False, True, False]
+
+
+def test_a_key_mean_of_another_size_is_refused():
+    """The kernel reads B*H*D values of it: a shorter one would be read past its end."""
+    from minimaxh3_amd import ops
+    k = torch.randn((2, 3, 40, 64), device="cuda", dtype=torch.bfloat16)
+    mean = ops.attn_kmean(k)
+    for bad in (mean[:1], mean[..., :32], mean.cpu()):
+        with pytest.raises(ValueError, match="mean must"):
+            ops.attn_quant_k(k, bad)
+    k8, sk = ops.attn_quant_k(k, mean)
+    k8f, skf = ops.attn_quant_k(k, mean.view(-1))
+    assert torch.equal(k8.view(torch.uint8), k8f.view(torch.uint8)) and torch.equal(sk, skf)
