@@ -222,6 +222,10 @@ class FP8Linear(nn.Module):
         With ``key_stats=False`` only the V statistics are taken (keys that are transformed
         after the projection, e.g. by a per-head norm or RoPE, need their own mean).
 
+        For long sequences: the projection keeps the tiles whose key sums it is defined by, and
+        below about 4000 tokens ``forward`` with a plain ``fp8_attention`` is as fast or faster (MI355X,
+        24 heads, both calls: 512 tokens 79 us chained, 51 separate; 2048 126 / 125; 20280 2679 / 2704).
+
         The output equals ``forward(x)`` bit for bit.  Where the statistics epilogue does not
         apply (LoRA adapters or an activation on this module, a non-bf16 input, S < 128, or
         heads x head_dim not a multiple of 256) stats is None, which ``fp8_attention`` takes
