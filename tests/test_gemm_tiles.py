@@ -128,3 +128,18 @@ def test_ring_depth_is_bounded_by_the_copy_counter(ring, fits):
                           "-I", build.CSRC, "-x", "hip", "-"], input=code, capture_output=True, text=True)
     assert (res.returncode == 0) == fits, res.stderr[-2000:]
     assert fits or "counts the copies" in res.stderr
+
+
+# (N, K, LoRA rank): tokens that take tiles 0 to 5 (test_gpu_gemm_ring.py compares their bits)
+EVERY_TILE = {
+    (3072, 2064, 0): (33, 201, 401, 701, 1301, 2701),
+    (2056, 3088, 32): (1, 299, 450, 1001, 2001, 4001),
+    (3072, 6160, 48): (1, 170, 331, 700, 1401, 2701),
+    (3072, 6160, 160): (1, 170, 331, 700, 1401, 2701),
+}
+
+
+@pytest.mark.parametrize("shape", EVERY_TILE)
+def test_every_tile_is_compared(pick, shape):
+    N, K, r = shape
+    assert [pick(m, N, K, r) for m in EVERY_TILE[shape]] == [0, 1, 2, 3, 4, 5]

@@ -8,6 +8,7 @@ import torch
 from oracle import linear as ol
 from oracle.numerics import bf16_round
 from tests.helpers import bf16_randn, to_gpu, with_outliers
+from tests.test_gemm_tiles import EVERY_TILE
 
 pytestmark = pytest.mark.gpu
 
@@ -58,6 +59,31 @@ def test_prefixes_have_the_same_bits_on_every_tile(N, K, r, gelu):
     full = gemm(M)
     for m in (1, 32, 65, 130, 300, 513, 1000, 2048, 3100):
         print(f"gemm prefix {m} N={N} K={K} r={r} gelu={gelu}", flush=True)
+        assert torch.equal(gemm(m), full[:m])
+
+
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("shape", EVERY_TILE)
+def test_every_tile_has_the_same_bits(shape, gelu):
+    """Prefixes of one x that take each of the six tiles, with ragged tokens, a K tail and a LoRA staged
+    in LDS or read from global memory."""
+    from minimaxh3_amd import ops
+    N, K, r = shape
+    rng = np.random.default_rng(N + K + r)
+    M = max(EVERY_TILE[shape])
+    _, _, b, (x8, sa), (w8, sw) = _operands(rng, M, N, K)
+    bias = to_gpu(b)
+    t = B = None
+    if r:
+        t, B = to_gpu(bf16_randn(rng, (M, r))), to_gpu(bf16_randn(rng, (N, r), 0.05))
+
+    def gemm(m):
+        return ops.gemm_rowwise(x8[:m], w8, sa[:m], sw.view(1, -1), bias, int(gelu), None if t is None else t[:m], B,
+                                0.75 if r else 0.0).view(torch.int16)
+
+    full = gemm(M)
+    for m in EVERY_TILE[shape]:
+        print(f"gemm tile {EVERY_TILE[shape].index(m)}: {m} x {N} x {K} r={r} gelu={gelu}", flush=True)
         assert torch.equal(gemm(m), full[:m])
 
 
